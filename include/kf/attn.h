@@ -79,7 +79,7 @@ typedef struct kf_attn_plan_t {
     int kv_per_split;      /* KV rows per partition                             */
     int grid_blocks;       /* workgroups of the main kernel                     */
     int block_threads;     /* threads per workgroup of the main kernel          */
-    size_t workspace_bytes;/* bytes kf_attn_fwd needs in `workspace`            */
+    size_t workspace_bytes;/* kf_attn_workspace_bytes()                          */
     int splits_per_block;  /* decode: KV partitions per workgroup (4 = the
                               short-split kernel, one partition per wave;
                               1 = the streaming decode kernel); 0 on prefill    */
@@ -114,11 +114,22 @@ int kf_attn_plan_for_cus(int B, int q_len, int kv_len, int H_q, int H_kv, int D,
 int kf_attn_kernel_names(int B, int q_len, int kv_len, int H_q, int H_kv, int D, int flags,
                          const int* kv_lens, char* buf, size_t buf_bytes);
 
-/* Bytes of device workspace kf_attn_fwd needs for this shape (0 when the
- * shape runs without split-KV partials: split decode and split prefill need
- * them).  Returns 0 for invalid shapes too;
- * kf_attn_plan reports why. */
+/* Bytes of device workspace with which kf_attn_fwd runs this shape its fastest
+ * (0 when the shape runs without split-KV partials: split decode and split
+ * prefill need them).  A decode whose heads do not divide over the compute
+ * units is shared evenly by all of their waves given this much; with less,
+ * down to num_splits partials of all query rows, it runs by the plan's splits
+ * (the two differ in the last bits, within the same tolerance).  Returns 0 for
+ * invalid shapes too; kf_attn_plan reports why. */
 size_t kf_attn_workspace_bytes(int B, int q_len, int kv_len, int H_q, int H_kv, int D);
+
+/* Bytes of workspace with which a kf_attn_fwd_ex call with kv_lens runs its
+ * fastest: at least kf_attn_workspace_bytes().  A large decode then shares the
+ * keys that the sequences really hold evenly over the compute units, instead
+ * of splitting every sequence by the kv_len rows allocated; a call given only
+ * kf_attn_workspace_bytes() still runs, by those splits (the two differ in
+ * the last bits, within the same tolerance).  No reference counterpart. */
+size_t kf_attn_workspace_bytes_lens(int B, int q_len, int kv_len, int H_q, int H_kv, int D);
 
 /* Attention forward, asynchronous on `stream`.
  *
@@ -186,7 +197,9 @@ int kf_attn_fwd_ex(const void* Q, const void* K, const void* V, void* O,
  * except a split prefill (KF_PATH_PREFILL_SPLIT), which is planned with as
  * many KV partitions as the scratch holds -- possibly fewer than
  * kf_attn_fwd_ex takes, in which case the results differ from its in the
- * last bits (both within the same tolerance of the exact result).
+ * last bits (both within the same tolerance of the exact result).  Likewise a
+ * decode whose even sharing (kf_attn_workspace_bytes, or _lens) needs more than
+ * the scratch runs by the plan's splits.
  * Every call on one device shares that device's array: calls that can run
  * concurrently on one device (two streams, two threads) race on it and must
  * be serialised by the caller; consecutive calls on one stream are safe.  The

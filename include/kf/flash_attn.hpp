@@ -162,9 +162,11 @@ inline hipError_t attn_fwd_ex(const uint16_t* Q, const uint16_t* K, const uint16
     kf_attn_plan_t plan;
     int st = kf_attn_plan(B, q_len, kv_len, H_q, H_kv, D, &plan);
     if (st != KF_OK) return status_to_hip(st);
+    const size_t need = kv_lens ? kf_attn_workspace_bytes_lens(B, q_len, kv_len, H_q, H_kv, D)
+                                : plan.workspace_bytes;
     void* ws = nullptr;
     size_t ws_bytes = 0;
-    hipError_t e = thread_workspace().get(stream, plan.workspace_bytes, &ws, &ws_bytes);
+    hipError_t e = thread_workspace().get(stream, need, &ws, &ws_bytes);
     if (e != hipSuccess) return e;
     st = kf_attn_fwd_ex(Q, K, V, O, Mi, Li, B, q_len, kv_len, H_q, H_kv, D, kv_lens, flags,
                         ws, ws_bytes, static_cast<void*>(stream));

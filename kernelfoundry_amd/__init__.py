@@ -39,7 +39,7 @@ __all__ = [
     "KF_ATTN_CAUSAL",
     "KF_ATTN_OUT_F16", "KF_ATTN_OUT_BF16", "KF_ATTN_LSE",
     "PATH_NAMES", "attn_fwd_ex_ptr", "attn_decode_paged", "attn_decode_paged_ptr",
-    "paged_workspace_bytes", "kernel_names",
+    "paged_workspace_bytes", "workspace_bytes_lens", "kernel_names",
 ]
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
@@ -137,6 +137,8 @@ def load_library(path: str = LIB_PATH):
     lib.kf_attn_plan_for_cus.restype = i
     lib.kf_attn_workspace_bytes.argtypes = [i] * 6
     lib.kf_attn_workspace_bytes.restype = sz
+    lib.kf_attn_workspace_bytes_lens.argtypes = [i] * 6
+    lib.kf_attn_workspace_bytes_lens.restype = sz
     lib.kf_attn_kernel_names.argtypes = [i] * 7 + [p, ctypes.c_char_p, sz]
     lib.kf_attn_kernel_names.restype = i
     lib.kf_attn_fwd.argtypes = [p, p, p, p, p, p] + [i] * 6 + [p, sz, p]
@@ -203,6 +205,11 @@ def kernel_names(B, q_len, kv_len, H_q, H_kv, D, causal=False, masked=False) -> 
 
 def workspace_bytes(B, q_len, kv_len, H_q, H_kv, D) -> int:
     return int(load_library().kf_attn_workspace_bytes(B, q_len, kv_len, H_q, H_kv, D))
+
+
+def workspace_bytes_lens(B, q_len, kv_len, H_q, H_kv, D) -> int:
+    """Workspace of a call with kv_lens (kf_attn_workspace_bytes_lens)."""
+    return int(load_library().kf_attn_workspace_bytes_lens(B, q_len, kv_len, H_q, H_kv, D))
 
 
 def attn_fwd_ptr(Q, K, V, O, Mi, Li, B, q_len, kv_len, H_q, H_kv, D, workspace=0,
@@ -274,15 +281,18 @@ def _output(torch, out, shape, out_dtype, device, stream):
     return out
 
 
-def _workspace(torch, workspace, need, device, stream):
+def _workspace(torch, workspace, need, device, stream, required=True):
     """The split-KV workspace: the caller's if it is a large enough buffer on
-    the device, else a new one (kept alive until ``stream`` passes it)."""
+    the device, else a new one (kept alive until ``stream`` passes it).  One
+    on another device is an error where the call cannot do without any
+    (``required``)."""
     if not need:
         return None
     if workspace is not None:
-        if workspace.device != device or not workspace.is_contiguous():
+        usable = workspace.device == device and workspace.is_contiguous()
+        if not usable and required:
             raise ValueError(f"workspace must be a contiguous tensor on {device}")
-        if workspace.numel() * workspace.element_size() >= need:
+        if usable and workspace.numel() * workspace.element_size() >= need:
             return workspace
     return _new(torch, need, torch.uint8, device, stream)
 
@@ -325,8 +335,12 @@ def attn_fwd(Q, K, V, out=None, *, return_stats=False, workspace=None, stream=No
         Mi = _new(torch, (B, H_q, q_len), torch.float32, Q.device, stream)
     if return_stats:
         Li = _new(torch, (B, H_q, q_len), torch.float32, Q.device, stream)
-    need = workspace_bytes(B, q_len, kv_len, H_q, H_kv, D)
-    workspace = _workspace(torch, workspace, need, Q.device, stream)
+    if kv_lens is None:
+        need, required = workspace_bytes(B, q_len, kv_len, H_q, H_kv, D), True
+    else:
+        need = workspace_bytes_lens(B, q_len, kv_len, H_q, H_kv, D)
+        required = workspace is None or workspace_bytes(B, q_len, kv_len, H_q, H_kv, D) > 0
+    workspace = _workspace(torch, workspace, need, Q.device, stream, required)
     if kv_lens is not None:
         # A contiguous copy would be made on torch's current stream, unordered
         # with a launch on another ``stream``: require the caller's layout.

@@ -90,6 +90,24 @@ constexpr int kWide256GroupKeys = 2 * kMinGroupKeys;
 // queries at 32 / 8 heads 1.08-1.09x (D = 64 1.02-1.06x), 2 x 4096 queries
 // against 6144 keys 1.09x, but 4 x 2048 queries 0.88x.
 constexpr int kWideCausalMinKeys = 2048;
+// Ragged decode (calls with key counts) against the capacity's splits, lengths
+// log-uniform over a factor of 16, paged, us before -> now at 32 / 8 heads,
+// D = 128: capacity 8 x 32768 keys 102 -> 55, 32 x 8192 90 -> 61, 16 x 4096
+// 30.7 -> 18.6, 6 x 4096 27.0 -> 14.8, but 4 x 4096 (2 stages per worker)
+// 13.6 -> 14.0; D = 64 12 x 2048 (2) 17.9 -> 12.5; D = 256, 16 / 4 heads,
+// 4 x 4096 (2) 18.9 -> 15.8.  16 rows (q_len 4) 16 x 4096 32.8 -> 26.6; with 32
+// rows (MQA) a partial is as large as a stage, and 64 x 4096 keys at D = 64
+// ran 13.6 -> 17.6: not taken.
+constexpr int kRaggedMinShare(int D) { return D == 128 ? 3 : 2; }
+constexpr int kRaggedMaxRows = 16;
+// Without key counts the split grid stays where it is one round of workgroups
+// (8 x 4096 keys 26.2 us against 28.6, 1 x 65536 47.2 against 52.7); a head
+// count that takes it several (each with its prologue and merge) goes to the
+// ragged decode: 12 x 4096 keys 44.1 -> 39.8, 20 x 4096 70.1 -> 60.3,
+// 40 x 1000 43.1 -> 35.4, 6 x 4096 29.8 -> 23.7; D = 256 (always two rounds)
+// 8 x 4096 at 16 / 4 heads 37.7 -> 31.7.  Of several rounds the least gain was
+// 24 x 8192 keys, 129.7 -> 130.3.
+constexpr int kRaggedEvenRows = 8;
 constexpr size_t kWsAlign = 256;
 
 thread_local int g_last_hip_error = 0;
@@ -151,6 +169,10 @@ struct Plan {
     int merge_per;      // split merge: splits per lane
     size_t ws_bytes;
     size_t ws_o_off, ws_m_off, ws_l_off;
+    int ragged_wgs;     // workgroups of the ragged decode (calls with key counts), 0 = none
+    size_t ragged_parts;  // its partials (two per worker) times rows
+    size_t ragged_bytes;  // its workspace: the partials and the heads' table
+    bool ragged_even;     // taken without key counts too
     int xcds;           // XCDs of the target device (workgroup id remap)
 };
 
@@ -231,6 +253,21 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
         p.merge_per = kf::merge_per_lane(p.merge_cw, p.n_splits);
         if (splits > 1 && rows_total * ((D / 4) / p.merge_cw) > INT_MAX) return KF_ERR_SIZE;
         p.path = splits > 1 ? KF_PATH_DECODE_SPLIT : KF_PATH_DECODE;
+        // Calls with key counts on a streaming job share the stages that the
+        // sequences really hold (kf_attn_decode_ragged_kernel; its stage
+        // numbers are ints), from kRaggedMinShare stages of capacity per
+        // worker and up to kRaggedMaxRows rows per KV head on.
+        const long long cap_stages = n_groups * ((kv_len + 31LL) / 32);
+        const int wgs = kf::ragged_workgroups(D, cus);
+        if (nst == 0 && R <= kRaggedMaxRows && cap_stages <= (1LL << 30) && rows_total * (D / 4) <= INT_MAX &&
+            cap_stages >= (long long)kRaggedMinShare(D) * wgs * kf::ragged_waves(D)) {
+            p.ragged_wgs = wgs;
+            p.ragged_parts = (size_t)2 * wgs * kf::ragged_waves(D) * (size_t)R;
+            p.ragged_bytes = split_ws_bytes(p.ragged_parts, D) + align_up((size_t)n_groups * sizeof(kf::u32x4), kWsAlign);
+            // Equal lengths: where the streaming kernel's grid takes more
+            // than one round of workgroups.
+            p.ragged_even = R <= kRaggedEvenRows && p.n_splits > 1 && p.grid > cus;
+        }
     } else {
         // Waves per workgroup: the most the head dimension allows.  When that
         // grid would leave CUs without a workgroup, D = 64 / 128 split each
@@ -360,6 +397,12 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
     }
     *pl = p;
     return KF_OK;
+}
+
+// The workspace with which a call runs its fastest; pl.ws_bytes is what it
+// cannot do without.
+size_t best_ws_bytes(const Plan& pl, bool lens) {
+    return (lens || pl.ragged_even) && pl.ragged_bytes > pl.ws_bytes ? pl.ragged_bytes : pl.ws_bytes;
 }
 
 inline bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
@@ -513,8 +556,25 @@ hipError_t launch_merge(const Plan& pl, const kf::AttnParams& prm, hipStream_t s
     return hipGetLastError();
 }
 
+// The ragged decode and its merge (one wave per query row and column block).
+template <int D>
+hipError_t launch_ragged(const Plan& pl, const kf::AttnParams& prm, hipStream_t stream) {
+    const dim3 grid(pl.ragged_wgs), block(kf::RaggedCfg<D>::kThreads);
+    if (prm.block_table)
+        kf::kf_attn_decode_ragged_kernel<D, true><<<grid, block, 0, stream>>>(prm);
+    else
+        kf::kf_attn_decode_ragged_kernel<D, false><<<grid, block, 0, stream>>>(prm);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    constexpr int kPerRow = (D / 4 + kf::kRaggedMergeCols - 1) / kf::kRaggedMergeCols, kWaves = kf::kRaggedMergeWaves;
+    const int blocks = (int)(((long long)pl.rows_total * kPerRow + kWaves - 1) / kWaves);
+    kf::kf_attn_ragged_merge_kernel<D><<<dim3(blocks), dim3(64 * kWaves), 0, stream>>>(prm);
+    return hipGetLastError();
+}
+
 template <int D>
 hipError_t launch_all(const Plan& pl, const kf::AttnParams& prm, hipStream_t stream) {
+    if (prm.ragged_heads) return launch_ragged<D>(pl, prm, stream);
     if (prefill_path(pl.path)) {
         const hipError_t e = launch_prefill_kernel<D>(pl, prm, stream);
         if (e != hipSuccess || pl.path != KF_PATH_PREFILL_SPLIT) return e;
@@ -571,7 +631,12 @@ int run(const Plan& pl, kf::AttnParams prm, const void* Q, const void* K, const 
         void* workspace, size_t workspace_bytes, void* stream) {
     const int st = check_args(flags, Q, K, V, O, prm.kv_lens, prm.block_table);
     if (st != KF_OK) return st;
-    if (pl.ws_bytes > 0) {
+    // The ragged decode, given a workspace that holds its partials (a smaller
+    // one, or none, runs the streaming kernel's plan).
+    const bool ragged = pl.ragged_wgs > 0 && (prm.kv_lens || pl.ragged_even) && workspace &&
+                        workspace_bytes >= pl.ragged_bytes && workspace_bytes >= pl.ws_bytes &&
+                        (reinterpret_cast<uintptr_t>(workspace) & (kWsAlign - 1)) == 0;
+    if (pl.ws_bytes > 0 && !ragged) {
         if (!workspace || workspace_bytes < pl.ws_bytes) return KF_ERR_WORKSPACE;
         if ((reinterpret_cast<uintptr_t>(workspace) & (kWsAlign - 1)) != 0) return KF_ERR_ALIGN;
     }
@@ -584,7 +649,18 @@ int run(const Plan& pl, kf::AttnParams prm, const void* Q, const void* K, const 
     prm.lse = (flags & KF_ATTN_LSE) ? 1 : 0;
     prm.Mi = row_max;
     prm.Li = row_sumexp;
-    if (pl.ws_bytes > 0) {
+    if (ragged) {
+        const size_t parts = pl.ragged_parts;
+        char* ws = static_cast<char*>(workspace);
+        prm.Opart = reinterpret_cast<float*>(ws);
+        ws += align_up(parts * D * sizeof(float), kWsAlign);
+        prm.Mpart = reinterpret_cast<float*>(ws);
+        ws += align_up(parts * sizeof(float), kWsAlign);
+        prm.Lpart = reinterpret_cast<float*>(ws);
+        ws += align_up(parts * sizeof(float), kWsAlign);
+        prm.ragged_heads = reinterpret_cast<kf::u32x4*>(ws);
+        prm.batch = pl.n_groups / H_kv;
+    } else if (pl.ws_bytes > 0) {
         char* ws = static_cast<char*>(workspace);
         prm.Opart = reinterpret_cast<float*>(ws + pl.ws_o_off);
         prm.Mpart = reinterpret_cast<float*>(ws + pl.ws_m_off);
@@ -686,7 +762,7 @@ int describe_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const 
     // run the 256-row kernel's grid at D = 64 / 128 and this grid at D = 256.
     plan->grid_blocks = pl.wide_row_tiles > 0 ? pl.wide_grid : pl.grid;
     plan->block_threads = pl.wide_row_tiles > 0 ? kf::WideCfg<128>::kThreads : pl.threads;
-    plan->workspace_bytes = pl.ws_bytes;
+    plan->workspace_bytes = best_ws_bytes(pl, false);
     plan->splits_per_block = prefill_path(pl.path) ? 0 : pl.short_stages > 0 ? kf::kShortWaves : 1;
     return KF_OK;
 }
@@ -732,9 +808,12 @@ int kf_attn_kernel_names(int B, int q_len, int kv_len, int H_q, int H_kv, int D,
     } else {
         if (pl.short_stages > 0)
             n = snprintf(tmp, sizeof(tmp), "kf_attn_decode_short_kernel<%d, %d>", D, pl.short_stages);
+        else if (pl.ragged_wgs > 0 && (kv_lens || pl.ragged_even))
+            n = snprintf(tmp, sizeof(tmp), "kf_attn_decode_ragged_kernel<%d, false> + kf_attn_ragged_merge_kernel<%d>",
+                         D, D);
         else
             n = snprintf(tmp, sizeof(tmp), "kf_attn_decode_kernel<%d, false>", D);
-        if (pl.path == KF_PATH_DECODE_SPLIT)
+        if (pl.path == KF_PATH_DECODE_SPLIT && !(pl.ragged_wgs > 0 && (kv_lens || pl.ragged_even)))
             n += snprintf(tmp + n, sizeof(tmp) - (size_t)n, " + kf_attn_split_merge_kernel<%d, %d, %d>", D,
                           pl.merge_per, pl.merge_cw);
     }
@@ -746,7 +825,7 @@ int kf_attn_kernel_names(int B, int q_len, int kv_len, int H_q, int H_kv, int D,
 size_t kf_attn_workspace_bytes(int B, int q_len, int kv_len, int H_q, int H_kv, int D) {
     Plan pl;
     if (make_plan(B, q_len, kv_len, H_q, H_kv, D, current_device_shape(), &pl) != KF_OK) return 0;
-    return pl.ws_bytes;
+    return best_ws_bytes(pl, false);
 }
 
 int kf_attn_fwd(const void* Q, const void* K, const void* V, float* O, float* row_max,
@@ -790,7 +869,7 @@ int kf_attn_fwd_noalloc(const void* Q, const void* K, const void* V, void* O, fl
     if (st != KF_OK) return st;
     if (pl.ws_bytes > kStaticScratchBytes) return KF_ERR_SCRATCH;
     void* ws = nullptr;
-    if (pl.ws_bytes > 0) {
+    if (best_ws_bytes(pl, kv_lens != nullptr) > 0) {
         hipError_t e = hipSuccess;
         ws = static_scratch(&e);
         if (!ws) return hip_fail(e);
@@ -798,10 +877,16 @@ int kf_attn_fwd_noalloc(const void* Q, const void* K, const void* V, void* O, fl
     kf::AttnParams prm{};
     prm.kv_lens = kv_lens;
     return run(pl, prm, Q, K, V, O, row_max, row_sumexp, q_len, kv_len, H_kv, D, flags, ws,
-               pl.ws_bytes, stream);
+               ws ? kStaticScratchBytes : 0, stream);
 }
 
 size_t kf_attn_noalloc_scratch_bytes(void) { return kStaticScratchBytes; }
+
+size_t kf_attn_workspace_bytes_lens(int B, int q_len, int kv_len, int H_q, int H_kv, int D) {
+    Plan pl;
+    if (make_plan(B, q_len, kv_len, H_q, H_kv, D, current_device_shape(), &pl) != KF_OK) return 0;
+    return best_ws_bytes(pl, true);
+}
 
 size_t kf_attn_decode_paged_workspace_bytes(int B, int q_len, int H_q, int H_kv, int D,
                                             int page_size, int max_pages_per_seq) {
@@ -811,7 +896,7 @@ size_t kf_attn_decode_paged_workspace_bytes(int B, int q_len, int H_q, int H_kv,
     if (make_plan(B, q_len, cap, H_q, H_kv, D, current_device_shape(), &pl, true) != KF_OK ||
         prefill_path(pl.path))
         return 0;
-    return pl.ws_bytes;
+    return best_ws_bytes(pl, true);
 }
 
 int kf_attn_decode_paged(const void* Q, const void* K_pages, const void* V_pages,

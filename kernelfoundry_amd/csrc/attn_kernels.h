@@ -1,6 +1,6 @@
 // attn_kernels.h -- gfx950 (CDNA4) flash-attention forward kernels.
 //
-// Four kernels, all hand-written for wave64 and the fp16 MFMA
+// All kernels are hand-written for wave64 and the fp16 MFMA
 // v_mfma_f32_32x32x16_f16:
 //
 //   kf_attn_prefill_kernel<D, kMask, NW>
@@ -23,6 +23,11 @@
 //                              one split of 32 or 64 keys and issues all of
 //                              its loads at once (one memory round trip);
 //                              the paged form reads K/V through a block table.
+//   kf_attn_decode_ragged_kernel<D, kPaged> / kf_attn_ragged_merge_kernel<D>
+//                              decode with key counts (and of head counts
+//                              that do not divide over the CUs): the waves
+//                              share the 32-key stages that the sequences
+//                              really hold evenly, across heads.
 //   kf_attn_split_merge_kernel<D, NPER, CW>
 //                              merges the split partials into O, Mi, Li.
 //
@@ -123,6 +128,9 @@ struct AttnParams {
     // XCDs of the device (8 on an MI355X in SPX mode, 1 per CPX partition):
     // the dispatcher deals workgroup ids round-robin over them.
     int xcds;
+    // Ragged decode (kf_attn_decode_ragged_kernel).
+    int batch;
+    u32x4* ragged_heads;     // [B * H_kv] where a head's partials are
 };
 
 enum : int { kOutF32 = 0, kOutF16 = 1, kOutBF16 = 2 };
@@ -234,6 +242,39 @@ __device__ __forceinline__ void qi_range(int r0, int r1, int q_len, int& lo, int
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ f32x16 mfma32(const f16x8& a, const f16x8& b, const f32x16& c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// Wait until at most N vector memory operations of this wave are outstanding.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    static_assert(N >= 0 && N < 64, "vmcnt");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// LDS-DMA of 16 bytes per lane into 1 KiB of LDS at `lds` (wave-uniform byte
+// address; lane l fills [16 l, 16 l + 16)), non-temporal, from base + off or
+// from a per-lane address.  As instructions of their own rather than the
+// builtin: the compiler answers the builtin with a wait for *every* copy in
+// flight before each LDS read of the array, where the kernel's own counted
+// waits (wait_vmcnt) leave the younger ones running.  They have no output
+// register; the caller waits before it reads the LDS and before it ends.
+// s_nop 4: the compiler keeps no hazard distances to instructions in asm, and
+// a VMEM instruction may read an SGPR no sooner than 5 wait states after a
+// VALU instruction (v_readfirstlane, v_readlane of a spilled register) wrote
+// it, and M0 no sooner than 1 after its write.
+__device__ __forceinline__ void lds_copy16_nt(uint32_t lds, const void* base, uint32_t off) {
+    // (The scalar base, also where the compiler does not see that it is one.)
+    const uint64_t b = (uint64_t)(uintptr_t)base;
+    base = (const void*)(uintptr_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(b >> 32)) << 32) |
+                                    (uint32_t)__builtin_amdgcn_readfirstlane((int)b));
+    lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds);
+    asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+                 ::"{m0}"(lds), "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void lds_copy16_nt(uint32_t lds, const void* lane_src) {
+    lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds);
+    asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, off nt"
+                 ::"{m0}"(lds), "v"(lane_src) : "memory");
 }
 
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -2137,6 +2178,612 @@ void kf_attn_decode_kernel(AttnParams p) {
                 p.Lpart[pi] = l;
             }
         }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Ragged decode: the streaming decode for calls with per-sequence key counts
+// (kv_lens, contiguous or paged).  A grid sized by the cache's capacity gives
+// every head the same splits, so a launch lasts as long as its longest
+// sequence and splits past a short sequence's keys do nothing.  Here the
+// 32-key stages that the sequences really hold are numbered head after head
+// (sequence-major: sequence b's H_kv heads have T_b = ceil(kvb / 32) stages
+// each) and every wave is a worker of its own that takes `share` consecutive
+// ones, so all CUs stream the same bytes whatever the lengths.  A worker's
+// share is cut into segments at head boundaries.  A segment that holds a
+// whole head writes its final rows.  The others are partials: a worker's last
+// segment is merged in LDS with those of the workgroup's other workers on the
+// same head, once, when all are done (a head inside one workgroup is final
+// then); a first segment whose head ends there, with others after it, goes to
+// memory as it is.  kf_attn_ragged_merge_kernel combines what is left.
+//
+// The bound is HBM.  K and V stages go HBM -> LDS by LDS-DMA into wave-private
+// slots (chunks XOR-swizzled by SwizzleRow<D>; V read back as V^T with
+// ds_read_b64_tr_b16): K(t + 1) is requested as soon as the score MFMAs have
+// read K(t), V(t + 1) as soon as the P.V MFMAs have read V(t), also across
+// segment boundaries, so a wave always has half a stage or more in flight
+// and holds none of it in registers.  Measured (32 / 8 heads, D = 128, paged,
+// contexts log-uniform from 512 to 8192 keys): 316 MB in 56 us, 5.6 TB/s
+// (90 us by the capacity's splits), and the merge 4.8.
+// Per-wave stamps of 16 x 4-row sequences: first copies requested 2 us after
+// entry (key counts, division, page ids), the stages at HBM rate, then 2 us
+// of LDS merge.
+// ---------------------------------------------------------------------------
+template <int D> struct RaggedCfg {
+    static constexpr int kWaves = D == 128 ? 8 : 4;     // workers per workgroup
+    static constexpr int kPerCU = D <= 64 ? 3 : 1;      // workgroups per CU (registers, LDS)
+    static constexpr int kThreads = 64 * kWaves;
+    static constexpr int kHalfBytes = kDecodeStage * D * 2;  // the K or V rows of a stage
+};
+// Workgroups for a device of `cus` compute units, and workers in each.
+inline int ragged_workgroups(int D, int cus) {
+    return cus * (D <= 64 ? RaggedCfg<64>::kPerCU : RaggedCfg<128>::kPerCU);
+}
+// Small jobs of few rows skip the merge in LDS: the waves' partials then cost
+// less memory traffic (R / 16 of a stage each, written and read) than the
+// workgroup's barrier and merge cost time (2.5 us), and one wave per
+// workgroup at a time spreads a job of few stages over all CUs.
+constexpr int kRaggedSpreadRows = 8;      // query rows per KV head
+constexpr int kRaggedSpreadStages = 12;   // stages per worker
+constexpr int kRaggedSpreadParts = 32;    // partials of an average head: one trip of the merge
+inline int ragged_waves(int D) { return D == 128 ? RaggedCfg<128>::kWaves : RaggedCfg<64>::kWaves; }
+
+// A wave-uniform element of an array that no kernel writes, by a scalar load
+// (the compiler falls back to a vector load, and its in-order wait for every
+// copy in flight, where the kernel's own stores might alias).
+__device__ __forceinline__ int uniform_load(const int* a, int i) {
+    return ((const __attribute__((address_space(4))) int*)a)[i];
+}
+
+// The kernel's parameter block re-read from the kernel arguments: for what a
+// long loop does not need, so that it holds no scalar registers there.
+// AttnParams is the kernel's only argument.
+__device__ __forceinline__ const AttnParams& late_params() {
+    auto ptr = (const __attribute__((address_space(4))) AttnParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(ptr));
+    return *(const AttnParams*)ptr;
+}
+
+// Keys of sequence b (0 past the batch) and 32-key stages for so many keys.
+__device__ __forceinline__ int seq_keys(const AttnParams& p, int b) {
+    return b >= p.batch ? 0 : p.kv_lens ? min(max(p.kv_lens[b], 0), p.kv_len) : p.kv_len;
+}
+__device__ __forceinline__ int key_stages(int keys) { return (keys + kDecodeStage - 1) / kDecodeStage; }
+
+// Inclusive prefix sum over the lanes.
+__device__ __forceinline__ int wave_scan(int v, int lane) {
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int u = __shfl_up(v, d);
+        if (lane >= d) v += u;
+    }
+    return v;
+}
+
+// n stages over parts of q stages, the first r of which take one more.
+struct StageSplit {
+    int n, q, r;
+    // Over m parts, as evenly as can be (part 0 has a stage if there is one).
+    static __device__ __forceinline__ StageSplit even(int n, int m) {
+        const int q = n / m;
+        return StageSplit{n, q, n - q * m};
+    }
+    __device__ __forceinline__ int first(int i) const { return min(i * q + min(i, r), n); }
+    __device__ __forceinline__ int part_of(int z) const {  // of stage z, 0 <= z < n
+        return z < r * (q + 1) ? z / (q + 1) : r + (z - r * (q + 1)) / max(q, 1);
+    }
+};
+
+// A run of consecutive stages of one head.
+struct RaggedSeg {
+    int b, h;     // sequence, KV head
+    int t0, n;    // first stage within the head, stages
+    int T, kvb;   // stages and keys of the head
+};
+
+// The stages of all sequences.  The first 64 sequences' keys and prefix sums
+// stay in registers, a lane each; larger batches re-read the others.
+struct RaggedMap {
+    int keys, inc;   // this lane's sequence: keys, stages per head up to and with it
+    int total;       // stages of all heads (the host keeps it within int)
+
+    __device__ __forceinline__ void init(const AttnParams& p, int lane) {
+        keys = seq_keys(p, lane);
+        inc = wave_scan(key_stages(keys), lane);
+        int sum = __builtin_amdgcn_readlane(inc, 63);
+        for (int b0 = 64; b0 < p.batch; b0 += 64)
+            sum += __builtin_amdgcn_readlane(wave_scan(key_stages(seq_keys(p, b0 + lane)), lane), 63);
+        total = sum * p.heads_kv;
+    }
+    // The segment that starts at global stage pos (pos < end <= total).
+    __device__ __forceinline__ RaggedSeg find(const AttnParams& p, int lane, int pos, int end) const {
+        RaggedSeg s{0, 0, 0, 0, 1, 0};
+        int k64 = keys, i64 = inc, carry = 0;
+        for (int b0 = 0;;) {
+            // Sequences whose stages all lie before pos come first.
+            const int k = __popcll(__ballot((carry + i64) * p.heads_kv <= pos));
+            if (k < 64) {
+                s.b = b0 + k;
+                s.kvb = __builtin_amdgcn_readlane(k64, k);
+                s.T = key_stages(s.kvb);
+                const int off = pos - (carry + __builtin_amdgcn_readlane(i64, k) - s.T) * p.heads_kv;
+                s.h = __builtin_amdgcn_readfirstlane(off / s.T);
+                s.t0 = off - s.h * s.T;
+                s.n = min(s.T - s.t0, end - pos);
+                return s;
+            }
+            carry += __builtin_amdgcn_readlane(i64, 63);
+            b0 += 64;
+            if (b0 >= p.batch) return s;  // not reached
+            k64 = seq_keys(p, b0 + lane);
+            i64 = wave_scan(key_stages(k64), lane);
+        }
+    }
+};
+
+template <int D, bool kPaged>
+__global__ __launch_bounds__(RaggedCfg<D>::kThreads, RaggedCfg<D>::kWaves * RaggedCfg<D>::kPerCU / 4)
+void kf_attn_decode_ragged_kernel(AttnParams p) {
+    using Cfg = RaggedCfg<D>;
+    using SW = SwizzleRow<D>;
+    constexpr int NW = Cfg::kWaves;
+    constexpr int kRowBytes = D * 2;
+    constexpr int kChunks = D / 8;                       // 16-byte chunks per row
+    constexpr int kHalf = Cfg::kHalfBytes;
+    constexpr int kInstr = kHalf / 1024;                 // LDS-DMA instructions per half stage
+    constexpr int kRowsPerInstr = 1024 / kRowBytes;
+    constexpr int kNKK = D / 16;                         // MFMA k-steps over D
+    constexpr int kNTD = (D < 32 ? 32 : D) / 32;         // 32-row O^T tiles
+    // A wave's slot: its K rows, then its V rows; after the loop its partial,
+    // [row][D] fp32.
+    __shared__ __attribute__((aligned(1024))) char slots[NW * 2 * kHalf];
+    static_assert(32 * D * 4 <= 2 * kHalf, "a partial fits the slot");
+    __shared__ float tail_m[NW * 32], tail_l[NW * 32];
+    __shared__ int tail_grp[NW], tail_slot[NW], tail_ends[NW];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 5;
+    const int row = lane & 31;
+    const int R = p.rows_per_group;
+    const int wg = blockIdx.x;
+    RaggedMap map;
+    map.init(p, lane);
+    // Merged: the stages go to the workgroups (as many as leave each of their
+    // waves one) and from them to their waves.
+    // Spread: straight to all waves, the first of every workgroup first.
+    const int workers = NW * (int)gridDim.x;
+    const bool spread = R <= kRaggedSpreadRows && map.total < kRaggedSpreadStages * workers &&
+                        p.batch * p.heads_kv >= workers / kRaggedSpreadParts;
+    const int worker = spread ? wave * (int)gridDim.x + wg : wg * NW + wave;
+    const StageSplit parts = spread ? StageSplit{map.total, (map.total + workers - 1) / workers, 0}
+                                    : StageSplit::even(map.total, max(min((int)gridDim.x, map.total / NW), 1));
+    int first_pos, end;
+    if (spread) {
+        first_pos = parts.first(worker);
+        end = parts.first(worker + 1);
+        if (first_pos >= end) return;  // wave-uniform: spread workers meet no barrier
+    } else {
+        const int wg_first = parts.first(wg), wg_stages = parts.first(wg + 1) - wg_first;
+        if (wg_stages <= 0) return;    // workgroup-uniform
+        const StageSplit waves = StageSplit::even(wg_stages, NW);
+        first_pos = wg_first + waves.first(wave);
+        end = wg_first + waves.first(wave + 1);
+    }
+
+    char* const ks = slots + wave * 2 * kHalf;
+    char* const vs = ks + kHalf;
+    const uint32_t ks_lds = (uint32_t)(uintptr_t)(lds_void*)ks, vs_lds = ks_lds + kHalf;
+
+    struct Stage {
+        size_t lo, hi;      // element offsets of rows 0..15 and 16..31
+        int k0, k1;         // first key; end of the keys (k1 - k0 rows are real)
+        int bad;            // invalid pages: bit 0 rows 0..15, bit 1 rows 16..31
+    };
+    // The ids of the page(s) of stage j of segment s: loads only, so that
+    // their latency can pass while the wave waits for something else.
+    struct PageIds {
+        int id0, id1;
+    };
+    auto page_ids = [&](const RaggedSeg& s, int j) {
+        PageIds ids{0, 0};
+        if constexpr (kPaged) {
+            const int k0 = (s.t0 + j) * kDecodeStage;
+            const int* tbl = p.block_table + (size_t)s.b * p.max_pages;
+            const int pi = k0 >> p.page_shift;
+            ids.id0 = uniform_load(tbl, pi);
+            // 16-row pages: the second half is the next page, if it has keys.
+            ids.id1 = uniform_load(tbl, p.page_shift == 4 && k0 + 16 < s.kvb ? pi + 1 : pi);
+        }
+        return ids;
+    };
+    auto stage_at = [&](const RaggedSeg& s, int j, const PageIds& ids) {
+        Stage st;
+        st.k0 = (s.t0 + j) * kDecodeStage;
+        st.k1 = min(s.kvb, st.k0 + kDecodeStage);
+        if constexpr (kPaged) {
+            const int sh = p.page_shift;
+            const bool ok0 = (unsigned)ids.id0 < (unsigned)p.num_pages;
+            const bool ok1 = (unsigned)ids.id1 < (unsigned)p.num_pages;
+            // An invalid page reads the pool's first page.
+            st.lo = ok0 ? ((((size_t)ids.id0 * p.heads_kv + s.h) << sh) + (size_t)(st.k0 & ((1 << sh) - 1))) * D : 0;
+            st.hi = sh != 4 ? (ok0 ? st.lo + 16 * D : 0) : ok1 ? (((size_t)ids.id1 * p.heads_kv + s.h) << 4) * D : 0;
+            st.bad = (ok0 ? 0 : 1) | (ok1 ? 0 : 2);
+        } else {
+            st.lo = ((size_t)(s.b * p.heads_kv + s.h) * p.kv_len + st.k0) * D;
+            st.hi = st.lo + 16 * D;
+            st.bad = 0;
+        }
+        return st;
+    };
+    // Lane l of instruction ii fills row ii * kRowsPerInstr + l / kChunks,
+    // physical chunk l % kChunks, which holds logical chunk
+    // (l % kChunks) ^ h(row); h depends on row & 15 only.
+    auto copy_half = [&](const uint16_t* base, const Stage& st, uint32_t dst) {
+        if (D >= 64 && st.k1 - st.k0 == kDecodeStage) {
+            const char* lo = reinterpret_cast<const char*>(base + st.lo);
+            const char* hi = reinterpret_cast<const char*>(base + st.hi);
+            const int lr = lane / kChunks;
+#pragma unroll
+            for (int ii = 0; ii < kInstr; ++ii) {
+                const int r = ii * kRowsPerInstr;        // rows of one half
+                lds_copy16_nt(dst + ii * 1024, (r >= 16 ? hi : lo) + (r & 15) * kRowBytes,
+                              (uint32_t)(lr * kRowBytes + (((lane % kChunks) ^ SW::h(r + lr)) % kChunks) * 16));
+            }
+        } else {
+            // The sequence's last stage: rows past its keys read the last one
+            // (finite data whose scores are masked).  The lane is opaque, so
+            // that none of this rare path's offsets live across the stages.
+            const int last = st.k1 - st.k0 - 1;
+            int ll = lane;
+            asm volatile("" : "+v"(ll));
+#pragma unroll
+            for (int ii = 0; ii < kInstr; ++ii) {
+                const int r = ii * kRowsPerInstr + ll / kChunks;
+                const int rc = min(r, last);
+                lds_copy16_nt(dst + ii * 1024,
+                              reinterpret_cast<const char*>(base + (rc >= 16 ? st.hi : st.lo) + (size_t)(rc & 15) * D) +
+                                  (((ll % kChunks) ^ SW::h(r)) % kChunks) * 16);
+            }
+        }
+    };
+
+    // LDS reads within a slot, as in the prefill kernels: K row l % 32,
+    // logical chunk 2 kk + l / 32; V^T by ds_read_b64_tr_b16 (16-lane group
+    // G = l / 16, w = l % 16).
+    const int hk = SW::h(row);
+    const int G = lane >> 4, w16 = lane & 15;
+    const int v_row = 4 * (G >> 1) + (w16 >> 2), v_d = 16 * (G & 1) + 4 * (w16 & 3);
+    f16x8 qf[kNKK];
+    f32x16 o[kNTD];
+    RowState st;
+    int lim_min, lim_lane;   // keys that every row, and this lane's row, sees
+    auto open_segment = [&](const RaggedSeg& c) {
+        const AttnParams& lp = late_params();
+        load_q_frags<D>(lp.Q + (size_t)(c.b * p.heads_kv + c.h) * R * D, row, R, lane, qf);
+        // Their wait belongs here, not to every stage's first use of them.
+#pragma unroll
+        for (int kk = 0; kk < kNKK; ++kk) asm volatile("" : "+v"(qf[kk]));
+        lim_min = lp.causal ? max(c.kvb - lp.q_len + 1, 0) : c.kvb;
+        lim_lane = row < R ? row_kv_limit(lp, c.kvb, row % lp.q_len) : c.kvb;
+        st = RowState{-INFINITY, -INFINITY, 0.f, -INFINITY};
+#pragma unroll
+        for (int td = 0; td < kNTD; ++td) o[td] = f32x16{};
+    };
+    // One stage, cs; with `more`, the next one, which it returns, is
+    // requested into the slots as they become free.
+    auto stage = [&](const Stage& cs, bool more, const RaggedSeg& nseg, int nj) {
+        const PageIds ids = page_ids(nseg, nj);
+        wait_vmcnt<kInstr>();  // K(t) has landed; V(t) may be in flight
+        f32x16 s[1];
+        s[0] = f32x16{};
+#pragma unroll
+        for (int kk = 0; kk < kNKK; ++kk) {
+            const int ko = row * kRowBytes + (((2 * kk + g) ^ hk) % kChunks) * 16;
+            const f16x8 a = *reinterpret_cast<const f16x8*>(ks + ko);
+            s[0] = mfma32(a, qf[kk], s[0]);
+        }
+        // K(t) has been read (the MFMAs consumed it): K(t + 1) may land.
+        __builtin_amdgcn_sched_barrier(0);
+        const Stage ns = stage_at(nseg, nj, ids);
+        if (more) copy_half(p.K, ns, ks_lds);
+        if (cs.k1 < cs.k0 + kDecodeStage || cs.k1 > lim_min || cs.bad) {
+            const int lim = min(cs.k1, lim_lane) - cs.k0;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int ar = acc_row(r, lane);
+                if (ar >= lim || (cs.bad >> (ar >> 4) & 1)) s[0][r] = -INFINITY;
+            }
+        }
+        f16x8 pb[2];
+        softmax_update<1, kNTD>(s, st, o, p.scale_log2, pb);
+
+        if (more)
+            wait_vmcnt<kInstr>();  // V(t) has landed; K(t + 1) may be in flight
+        else
+            wait_vmcnt<0>();
+        if (kPaged && cs.bad) {
+            // V rows of an invalid page -> zeros, so that P = 0 meets finite
+            // values.  Rows past the keys repeat the last key's.
+            const int last = cs.k1 - cs.k0 - 1;
+            for (int i = lane; i < kDecodeStage * kChunks; i += 64) {
+                const int r = min(i / kChunks, last);
+                if (cs.bad >> (r >> 4) & 1) *reinterpret_cast<u32x4*>(vs + i * 16) = u32x4{0u, 0u, 0u, 0u};
+            }
+            wave_lds_sync();
+        }
+#pragma unroll
+        for (int td = 0; td < kNTD; ++td) {
+            // D = 16: the groups with d >= 16 give the zero rows 16..31 of V^T.
+            const int d = 32 * td + v_d;
+            const bool dok = d < D;
+            const int dc = dok ? d : d - 16;
+            int voff[2];
+#pragma unroll
+            for (int h2 = 0; h2 < 2; ++h2) {
+                const int r = v_row + 8 * h2;
+                voff[h2] = r * kRowBytes + (((dc >> 3) ^ SW::h(r)) % kChunks) * 16 + ((dc >> 2) & 1) * 8;
+            }
+#pragma unroll
+            for (int jj = 0; jj < 2; ++jj) {
+                const f16x4 lo = lds_read_tr16(vs + voff[0] + jj * 16 * kRowBytes);
+                const f16x4 hi = lds_read_tr16(vs + voff[1] + jj * 16 * kRowBytes);
+                f16x8 a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                if (D < 32 && !dok) a = f16x8{};
+                o[td] = mfma32(a, pb[jj], o[td]);
+            }
+        }
+        // V(t) has been read: V(t + 1) may land.
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) copy_half(p.V, ns, vs_lds);
+        return ns;
+    };
+
+    int tgrp = -1, tslot = 0, tends = 0;  // the worker's partial last segment
+    if (first_pos < end) {
+        int pos = first_pos;     // global stage at which `cur` starts
+        RaggedSeg cur = map.find(p, lane, pos, end);
+        Stage cs = stage_at(cur, 0, page_ids(cur, 0));
+        copy_half(p.K, cs, ks_lds);
+        copy_half(p.V, cs, vs_lds);
+        open_segment(cur);
+        int j = 0;
+        for (int left = end - first_pos; left > 0; --left) {
+            const bool seg_end = j + 1 == cur.n;
+            // The stage after this one; past the segment's last it is the
+            // next head's first, or the next sequence's that has keys (after
+            // the share's last, this one again, not requested).
+            RaggedSeg nxt = cur;
+            if (seg_end && left > 1) {
+                const int npos = pos + cur.n;
+                if (cur.h + 1 < p.heads_kv)
+                    nxt = RaggedSeg{cur.b, cur.h + 1, 0, min(cur.T, end - npos), cur.T, cur.kvb};
+                else
+                    nxt = map.find(p, lane, npos, end);
+            }
+            cs = stage(cs, left > 1, nxt, left == 1 ? j : seg_end ? 0 : j + 1);
+            ++j;
+            if (!seg_end) continue;
+
+            const AttnParams& lp = late_params();
+            const int grp = cur.b * p.heads_kv + cur.h;
+            const int slot = 2 * worker + (pos != first_pos ? 1 : 0);
+            const bool whole = cur.n == cur.T;
+            // The worker of a head's first stage tells the merge where the
+            // head's partials are: the first slot, how many such follow each
+            // other at a stride (1: the rows are final unless one more is
+            // alone), the slot of one that went to memory by itself or -1,
+            // the stride.
+            if (cur.t0 == 0 && lane == 0) {
+                const int z = pos + cur.T;                  // end of the head
+                const int ep = parts.part_of(z - 1);        // part of its last stage
+                int groups = spread ? ep - worker + 1 : 1;
+                uint32_t alone = ~0u;
+                if (!spread && !whole) {
+                    const int elo = parts.first(ep);
+                    const StageSplit ew = StageSplit::even(parts.first(ep + 1) - elo, NW);
+                    const int ewave = ew.part_of(z - 1 - elo);
+                    const bool tail = z == elo + ew.first(ewave + 1);  // that wave's last segment
+                    groups = ep - wg + (tail || ewave > 0 ? 1 : 0);
+                    if (!tail) alone = 2 * (ep * NW + ewave);
+                }
+                lp.ragged_heads[grp] = u32x4{(uint32_t)slot, (uint32_t)groups, alone, spread ? 2u : 2u * NW};
+            }
+            if (!whole && left == 1 && !spread) {
+                tgrp = grp;
+                tslot = slot;
+                tends = (cur.t0 == 0 ? 1 : 0) | (cur.t0 + cur.n == cur.T ? 2 : 0);
+            } else {
+                // A whole head's final rows, or the partial of a head that
+                // ended with this worker's first segment.
+                const float l = sum_xor32(st.l);
+                const bool none = st.rmax == -INFINITY;
+                const float beta = none ? 0.f : rebase_factor(st.m, st.rmax, lp.scale_log2);
+                const float m_nat = none ? -INFINITY : st.rmax * lp.scale;
+                int el = lane;  // opaque: no store address lives across the stages
+                asm volatile("" : "+v"(el));
+                const int erow = el & 31, eg = el >> 5;
+                if (erow < R) {
+                    const size_t ri = (size_t)grp * R + erow, pi = (size_t)slot * R + erow;
+                    if (whole) {
+                        store_o_row_any<D>(lp, ri, o, l > 0.f ? 1.0f / l : 0.f, eg);
+                        if (eg == 0) store_stats(lp, ri, m_nat, l * beta);
+                    } else {
+                        store_o_row<kOutPartial, D>(lp, pi, o, beta, eg);
+                        if (eg == 0) {
+                            lp.Mpart[pi] = m_nat;
+                            lp.Lpart[pi] = l * beta;
+                        }
+                    }
+                }
+            }
+            if (left > 1) {
+                pos += cur.n;
+                cur = nxt;
+                j = 0;
+                open_segment(cur);
+            }
+        }
+    }
+
+    if (spread) return;
+    // ---- The workers' last segments, merged per head. ----
+    const AttnParams& lp = late_params();
+    if (tgrp >= 0) {
+        const float l = sum_xor32(st.l);
+        const bool none = st.rmax == -INFINITY;
+        const float beta = none ? 0.f : rebase_factor(st.m, st.rmax, lp.scale_log2);
+        if (row < R) {
+            float* dst = reinterpret_cast<float*>(ks) + row * D;
+#pragma unroll
+            for (int td = 0; td < kNTD; ++td)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int d = 32 * td + 8 * i + 4 * g;
+                    // Chunks XOR-ed by the row, against bank conflicts.
+                    if (d < D)
+                        *reinterpret_cast<f32x4*>(dst + ((d / 4) ^ (row & (D / 4 - 1) & 7)) * 4) =
+                            f32x4{o[td][4 * i], o[td][4 * i + 1], o[td][4 * i + 2], o[td][4 * i + 3]} * beta;
+                }
+            if (g == 0) {
+                tail_m[wave * 32 + row] = none ? -INFINITY : st.rmax * lp.scale;
+                tail_l[wave * 32 + row] = l * beta;
+            }
+        }
+    }
+    if (lane == 0) {
+        tail_grp[wave] = tgrp;
+        tail_slot[wave] = tslot;
+        tail_ends[wave] = tends;
+    }
+    __syncthreads();
+    // Runs of workers on one head: bit w of `live` where worker w has a
+    // partial, of `heads` where a run starts (a worker without one ends it).
+    const int tg = lane < NW ? tail_grp[lane] : -1;
+    const int tg_before = __shfl_up(tg, 1);
+    const uint32_t live = (uint32_t)__ballot(tg >= 0);
+    const uint32_t heads = (uint32_t)__ballot(tg >= 0 && (lane == 0 || tg != tg_before));
+    for (uint32_t left = heads; left;) {
+        const int w0 = __builtin_ctz(left);
+        left &= left - 1;
+        const uint32_t run = live & ((left ? left & -left : 1u << NW) - 1) & ~((1u << w0) - 1);
+        const int w1 = w0 + __builtin_popcount(run);  // past the run's last
+        const int grp = __builtin_amdgcn_readlane(tg, w0);
+        // The run holds the whole head: final rows.
+        const bool whole = ((tail_ends[w0] & 1) != 0) && ((tail_ends[w1 - 1] & 2) != 0);
+        const int slot = tail_slot[w0];
+        for (int i = tid; i < R * (D / 4); i += Cfg::kThreads) {
+            const int mrow = i / (D / 4), c = i % (D / 4);
+            float mw[NW], lw[NW];
+            f32x4 ow[NW];
+            // Every worker's, so that the loads are in flight together; those
+            // outside the run count for nothing.
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const bool in = w >= w0 && w < w1;
+                mw[w] = in ? tail_m[w * 32 + mrow] : -INFINITY;
+                lw[w] = tail_l[w * 32 + mrow];
+                ow[w] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(slots + w * 2 * kHalf) +
+                                                        mrow * D + (c ^ (mrow & (D / 4 - 1) & 7)) * 4);
+            }
+            float m = mw[0];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) m = fmaxf(m, mw[w]);
+            float l = 0.f;
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < NW; ++w)
+                if (mw[w] != -INFINITY) {
+                    const float wt = exp2_hw((mw[w] - m) * kLog2e);
+                    l += wt * lw[w];
+                    acc += wt * ow[w];
+                }
+            const size_t ri = (size_t)grp * R + mrow, pi = (size_t)slot * R + mrow;
+            if (whole) {
+                store_out4(lp, ri * D + 4 * c, acc * (l > 0.f ? 1.0f / l : 0.f));
+                if (c == 0) store_stats(lp, ri, m, l);
+            } else {
+                *reinterpret_cast<f32x4*>(lp.Opart + pi * D + 4 * c) = acc;
+                if (c == 0) {
+                    lp.Mpart[pi] = m;
+                    lp.Lpart[pi] = l;
+                }
+            }
+        }
+    }
+}
+
+// Merge of the ragged decode's partials: one wave per (query row, block of CW
+// float4 columns), 64 / CW split lanes.  A head's partials are the one of the
+// worker (spread) or the merged one of the workgroup where it starts, one of
+// each further worker or workgroup (in its first worker's slot), and at most
+// one that a workgroup's worker wrote by itself.
+// A head whose rows are final is left; a sequence without keys gets O = 0,
+// Mi = -inf, Li = 0 here.
+constexpr int kRaggedMergeCols = 8;
+constexpr int kRaggedMergeWaves = 4;
+template <int D>
+__global__ __launch_bounds__(64 * kRaggedMergeWaves)
+void kf_attn_ragged_merge_kernel(AttnParams p) {
+    constexpr int CW = D / 4 < kRaggedMergeCols ? D / 4 : kRaggedMergeCols;
+    constexpr int kNCB = (D / 4) / CW;                // column blocks per row
+    constexpr int kSL = 64 / CW;                      // split lanes per column
+    constexpr int kUnroll = 4;
+    const int lane = threadIdx.x & 63;
+    const int wid = blockIdx.x * kRaggedMergeWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ri = wid / kNCB, cb = wid % kNCB;
+    if (ri >= p.rows_total) return;
+    const int R = p.rows_per_group;
+    const int grp = ri / R, r = ri - grp * R;
+    const u32x4 head = p.ragged_heads[grp];           // not written for a sequence without keys
+    const bool empty = seq_keys(p, grp / p.heads_kv) == 0;
+    const int groups = empty ? 0 : (int)head.y;
+    const int ns = empty ? 0 : groups + ((int)head.z >= 0 ? 1 : 0);
+    if (ns == 1) return;
+    const int stride = (int)head.w, first = (int)head.x / max(stride, 1);
+    const int c = cb * CW + lane % CW, sl = lane / CW;
+
+    float m = -INFINITY, l = 0.f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = sl; k0 < ns; k0 += kSL * kUnroll) {
+        f32x4 ov[kUnroll];
+        float mv[kUnroll], lv[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const int k = min(k0 + u * kSL, ns - 1);
+            const int slot = k == 0 ? (int)head.x : k < groups ? (first + k) * stride : (int)head.z;
+            const size_t pi = (size_t)slot * R + r;
+            ov[u] = *reinterpret_cast<const f32x4*>(p.Opart + pi * D + 4 * c);
+            mv[u] = p.Mpart[pi];
+            lv[u] = p.Lpart[pi];
+        }
+        float mx = m;
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) mx = fmaxf(mx, mv[u]);
+        if (mx == -INFINITY) continue;
+        const float keep = exp2_hw((m - mx) * kLog2e);
+        acc *= keep;
+        l *= keep;
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const float w = k0 + u * kSL < ns ? exp2_hw((mv[u] - mx) * kLog2e) : 0.f;
+            l += w * lv[u];
+            acc += w * ov[u];
+        }
+        m = mx;
+    }
+    const float mm = reduce_mod<CW, true>(m);
+    const float w = mm == -INFINITY ? 0.f : exp2_hw((m - mm) * kLog2e);
+    l = reduce_mod<CW, false>(l * w);
+    acc *= w;
+    acc.x = reduce_mod<CW, false>(acc.x);
+    acc.y = reduce_mod<CW, false>(acc.y);
+    acc.z = reduce_mod<CW, false>(acc.z);
+    acc.w = reduce_mod<CW, false>(acc.w);
+    if (sl == 0) {
+        store_out4(p, (size_t)ri * D + 4 * c, acc * (l > 0.f ? 1.0f / l : 0.f));
+        if (c == 0) store_stats(p, ri, mm, l);
     }
 }
 

@@ -1,0 +1,169 @@
+"""Ragged decode (kf_attn_decode_ragged_kernel): decode with key counts whose
+waves share the stages that the sequences really hold.
+
+Shapes where the division can go wrong: empty sequences and single keys, one
+long sequence among short ones (a head over many workers), hundreds of heads
+inside one worker's share, more than 64 sequences (the batch map's second
+round), counts past the capacity, 1 to 16 rows per KV head (both ways of
+merging), every head dimension, page sizes from 16 rows, invalid page ids.
+Bar as in the other parity tests (fp64 oracle), and the same call by the
+capacity's splits (a workspace of only kf_attn_workspace_bytes) within 2e-4:
+P is rounded to fp16 against other row maxima, 2^-11 of values of order 1.
+"""
+import numpy as np
+import pytest
+
+import kernelfoundry_amd as kf
+from oracle import attn_oracle as orc
+
+
+def _lens(kind, B, cap, seed):
+    rng = np.random.default_rng(seed)
+    if kind == "one_long":
+        n = rng.integers(0, 40, B)
+        n[B // 2] = cap
+    elif kind == "short":
+        n = rng.integers(1, 70, B)
+    elif kind == "full":
+        n = np.full(B, cap)
+    elif kind == "empty":
+        n = np.zeros(B)
+    else:
+        n = np.exp(rng.uniform(np.log(cap / 16), np.log(cap), B))
+        n[:3] = (0, 1, cap + 9)  # none, one key, clamped
+    return n.astype(np.int32)
+
+
+CASES = [
+    # B, H_q, H_kv, q_len, cap, D, page_size (0: contiguous), lengths, causal
+    (16, 32, 8, 1, 4096, 128, 0, "mixed", False),
+    (16, 32, 8, 4, 4096, 128, 0, "mixed", True),       # 16 rows: merged in LDS
+    (32, 32, 8, 1, 8192, 128, 16, "one_long", False),
+    (70, 8, 8, 2, 2048, 128, 64, "mixed", True),       # > 64 sequences
+    (130, 8, 4, 1, 1024, 128, 32, "short", False),
+    (16, 32, 8, 1, 4096, 128, 16, "full", False),
+    (16, 32, 8, 1, 4096, 128, 16, "empty", False),
+    (24, 16, 16, 1, 2048, 64, 128, "mixed", False),
+    (20, 32, 4, 2, 3000, 64, 0, "one_long", True),     # 16 rows, ragged capacity
+    (64, 16, 16, 1, 4000, 16, 0, "mixed", False),
+    (96, 4, 2, 3, 4096, 16, 16, "one_long", True),
+    (16, 16, 4, 1, 4096, 256, 16, "mixed", False),
+    (16, 16, 4, 3, 4096, 256, 0, "one_long", True),    # 12 rows
+]
+
+
+def _id(c):
+    return "B{}_Hq{}_Hkv{}_q{}_cap{}_D{}_ps{}_{}".format(*c[:8])
+
+
+@pytest.mark.parametrize("case", CASES, ids=_id)
+def test_cases_take_the_ragged_kernel(case):
+    B, H_q, H_kv, q, cap, D, ps, kind, causal = case
+    cap = -(-cap // ps) * ps if ps else cap
+    names = kf.kernel_names(B, q, cap, H_q, H_kv, D, causal=causal, masked=True)
+    assert names == f"kf_attn_decode_ragged_kernel<{D}, false> + kf_attn_ragged_merge_kernel<{D}>"
+    assert kf.workspace_bytes_lens(B, q, cap, H_q, H_kv, D) >= kf.workspace_bytes(B, q, cap, H_q, H_kv, D)
+    if ps:
+        assert kf.paged_workspace_bytes(B, q, H_q, H_kv, D, ps, cap // ps) == \
+            kf.workspace_bytes_lens(B, q, cap, H_q, H_kv, D)
+
+
+def test_other_calls_keep_their_kernels_and_workspace():
+    # Equal lengths take it where the split grid is several rounds of
+    # workgroups (96 heads, not 64 or 128), and are asked for its workspace.
+    assert "ragged" in kf.kernel_names(12, 1, 4096, 32, 8, 128)
+    assert kf.workspace_bytes(12, 1, 4096, 32, 8, 128) == kf.workspace_bytes_lens(12, 1, 4096, 32, 8, 128)
+    for B in (8, 16, 32):
+        assert "ragged" not in kf.kernel_names(B, 1, 4096, 32, 8, 128)
+    # Small capacities and more than 16 rows per KV head never.
+    for shape in ((4, 1, 4096, 32, 8, 128), (1, 1, 4096, 32, 8, 128), (64, 1, 4096, 32, 1, 64)):
+        assert "ragged" not in kf.kernel_names(*shape, masked=True)
+        assert kf.workspace_bytes_lens(*shape) == kf.workspace_bytes(*shape)
+    # A workspace of the capacity's plan is enough (the call then ends at
+    # its first HIP call on a host without a GPU), one byte less is not.
+    import torch
+    if torch.cuda.is_available():
+        return
+    fake, ws = 1 << 20, 1 << 24
+    for B in (16, 32):
+        need = kf.workspace_bytes(B, 1, 4096, 32, 8, 128)
+        for flags in (0, kf.KF_ATTN_LSE):
+            def call(n, w=ws):
+                return kf.attn_fwd_ex_ptr(fake, fake, fake, fake, 0, 0, B, 1, 4096, 32, 8, 128,
+                                          kv_lens=fake, flags=flags, workspace=w, workspace_bytes=n)
+            assert call(need) == kf.KF_ERR_HIP
+            assert call(kf.workspace_bytes_lens(B, 1, 4096, 32, 8, 128)) == kf.KF_ERR_HIP
+            if need:
+                assert call(need - 1) == kf.KF_ERR_WORKSPACE
+                assert call(need, ws + 16) == kf.KF_ERR_ALIGN
+            else:
+                assert call(0, 0) == kf.KF_ERR_HIP
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=_id)
+def test_ragged_parity(case):
+    import torch
+    B, H_q, H_kv, q, cap, D, ps, kind, causal = case
+    cap = -(-cap // ps) * ps if ps else cap
+    print("case", case, flush=True)
+    lens = _lens(kind, B, cap, 11 + B)
+    rng = np.random.default_rng(B + D)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    q16 = rng.standard_normal((B, H_q, q, D), dtype=np.float32).astype(np.float16)
+    Q, L = dev(q16), dev(lens)
+    used = np.minimum(lens, cap)
+    if ps:
+        need = -(-used // ps)
+        pool = int(need.sum()) + 5
+        kp, vp = (rng.standard_normal((pool, H_kv, ps, D), dtype=np.float32).astype(np.float16)
+                  for _ in range(2))
+        table = np.full((B, cap // ps), -1, dtype=np.int32)
+        ids, at = rng.permutation(pool), 0
+        for b in range(B):
+            table[b, :need[b]] = ids[at:at + need[b]]
+            at += need[b]
+        for b in rng.integers(0, B, 3):      # pages that do not exist
+            if need[b] > 1:
+                table[b, rng.integers(0, need[b])] = pool + 3
+        K, V, T = dev(kp), dev(vp), dev(table)
+        O, Mi, Li = kf.attn_decode_paged(Q, K, V, T, L, return_stats=True, causal=causal)
+        O16, lse = kf.attn_decode_paged(Q, K, V, T, L, out_dtype=torch.float16, return_lse=True,
+                                        causal=causal)
+        kc, valid = orc.paged_to_contiguous(kp, table, ps)
+        vc, _ = orc.paged_to_contiguous(vp, table, ps)
+        by_capacity = None
+    else:
+        kc, vc = (rng.standard_normal((B, H_kv, cap, D), dtype=np.float32).astype(np.float16)
+                  for _ in range(2))
+        K, V, valid = dev(kc), dev(vc), None
+        O, Mi, Li = kf.attn_fwd(Q, K, V, return_stats=True, causal=causal, kv_lens=L)
+        O16, lse = kf.attn_fwd(Q, K, V, out_dtype=torch.float16, return_lse=True, causal=causal, kv_lens=L)
+        # The same by the capacity's splits.
+        n = kf.workspace_bytes(B, q, cap, H_q, H_kv, D)
+        ws = torch.empty(max(n, 256), dtype=torch.uint8, device="cuda")
+        by_capacity = torch.empty_like(O)
+        st = kf.attn_fwd_ex_ptr(Q.data_ptr(), K.data_ptr(), V.data_ptr(), by_capacity.data_ptr(), 0, 0, B, q,
+                                cap, H_q, H_kv, D, kv_lens=L.data_ptr(),
+                                flags=kf.KF_ATTN_CAUSAL if causal else 0, workspace=ws.data_ptr(),
+                                workspace_bytes=n, stream=torch.cuda.current_stream().cuda_stream)
+        assert st == kf.KF_OK
+    torch.cuda.synchronize()
+    Or, Mr, Lr = orc.sdpa(q16, kc, vc, causal=causal, kv_lens=[int(x) for x in used],
+                          **({"key_valid": valid} if valid is not None else {}))
+    if by_capacity is not None:
+        assert (O - by_capacity).abs().max().item() <= 2e-4 * max(1.0, np.abs(Or).max())
+    O, Mi, Li, lse = (x.cpu().numpy() for x in (O, Mi, Li, lse))
+    assert np.isfinite(O).all()
+    empty = np.isneginf(Mr)
+    assert np.array_equal(np.isneginf(Mi), empty) and np.array_equal(np.isneginf(lse), empty)
+    assert (O[empty] == 0).all() and (Li[empty] == 0).all()
+    full = ~empty
+    if full.any():
+        ok, max_abs, rel = orc.within_tolerance(O, Or)
+        assert ok, f"max_abs={max_abs:.3g} rel={rel:.3g}"
+        assert np.abs(Mi[full] - Mr[full]).max() <= 1e-4
+        assert np.abs(Li[full] / Lr[full] - 1).max() <= 1e-3
+        assert np.abs(lse[full] - (Mr[full] + np.log(Lr[full]))).max() <= 1e-3
+    # The same rows, rounded once.
+    assert np.array_equal(O16.cpu().numpy(), O.astype(np.float16))
