@@ -11,6 +11,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <numeric>
 
 #include "attn_kernels.h"
 #include "kf/attn.h"
@@ -108,6 +109,8 @@ constexpr int kRaggedMaxRows = 16;
 // 8 x 4096 at 16 / 4 heads 37.7 -> 31.7.  Of several rounds the least gain was
 // 24 x 8192 keys, 129.7 -> 130.3.
 constexpr int kRaggedEvenRows = 8;
+constexpr int kCausalShortKeys = 768;
+constexpr int kCausalWide2Keys = 1024;
 constexpr size_t kWsAlign = 256;
 
 thread_local int g_last_hip_error = 0;
@@ -164,6 +167,11 @@ struct Plan {
     int wide_grid;      // workgroups of the wide kernel
     int wide_kv_groups; // KV groups of the wide kernel (2: D = 256, 128 rows per workgroup)
     bool wide_causal;   // D = 64 / 128: causal calls take the wide kernel too
+    // Unsplit causal calls that take neither that nor the plan above (0 waves:
+    // they take it): waves, KV groups, the groups the 8-wave kernel makes of
+    // one (kf_attn_prefill_kernel), and the 128-row KV-group kernel at D = 256.
+    int causal_waves, causal_kv_groups, causal_groups;
+    bool causal_wide2;
     int short_stages;   // decode: 32-key stages per split of the short-split kernel, 0 = streaming kernel
     int merge_cw;       // split merge: float4 columns per wave
     int merge_per;      // split merge: splits per lane
@@ -186,6 +194,47 @@ size_t split_ws_bytes(size_t parts, int D) {
 }
 
 bool prefill_path(int path) { return path == KF_PATH_PREFILL || path == KF_PATH_PREFILL_SPLIT; }
+
+// The layout of an unsplit causal call where the unmasked one's is not the
+// best: a row sees kv_len - q_len / 2 keys on average against kv_len at most,
+// and the rows of a large tile end at different keys.
+void plan_causal(Plan& p, int q_len, int kv_len, int D, int cus) {
+    const long long avg_keys = (long long)kv_len - q_len / 2;
+    const auto grid_of = [&](int rows) { return (long long)p.n_groups * ((p.R + rows - 1) / rows); };
+    if (D >= 256) {
+        // 256-row tiles that leave CUs idle, all in one round as long as its
+        // longest tile: 128-row tiles in two KV groups, longest first, halve
+        // that chain (16 / 4 heads: 2 x 1500 queries 87.7 -> 72 us, 1 x 3000
+        // 149 -> 117; 3 x 1000 61.3 -> 58.8 and 4 x 600 44.6 -> 42.4 are left
+        // as they are).  A full round keeps the 256-row tiles, as unmasked
+        // calls do (1 x 4096: 204 against 179).
+        p.causal_wide2 = p.wide_row_tiles > 0 && p.wide_kv_groups == 1 && p.wide_grid < cus &&
+                         kv_len >= kCausalWide2Keys && grid_of(128) <= INT_MAX;
+        return;
+    }
+    // (Calls with fewer keys than queries, whose first rows see none, stay.)
+    if (D < 64 || p.waves != 8 || p.kv_groups != 1 || p.wide_causal || kv_len < q_len) return;
+    // One round of 256-row tiles: two KV groups inside the 8-wave kernel
+    // (figures there), unless the rows see nearly all keys or so few that
+    // the second round's prologue costs more (2 x 1024 queries 37.6 -> 38.7
+    // us, 4 x 512 25.9 -> 31.5).
+    if (p.grid <= cus && q_len % 256 == 0) {
+        if (avg_keys >= kCausalShortKeys && 5 * avg_keys <= 4LL * kv_len && grid_of(128) <= INT_MAX)
+            p.causal_groups = 2;
+        return;
+    }
+    // 256-row tiles that straddle heads, or that few keys make short: 4-wave
+    // workgroups, 128 rows each (D = 64: 64 rows in two KV groups), of which a
+    // CU holds two (three).  32 / 8 heads, D = 128: 2200 queries 80 -> 75 us,
+    // 3000 113 -> 109, 3 x 1000 60.2 -> 54.2, 2 x 3000 205 -> 197, 4 x 1024
+    // 69.6 -> 64.6, but 2 x 2048 98.4 -> 97.8 and 4096 165 -> 170; D = 64:
+    // 3000 78.5 -> 71, 2 x 1000 31.3 -> 27.0.
+    const bool straddle = q_len % 256 != 0;
+    if (avg_keys < (straddle ? kWideCausalMinKeys : kCausalShortKeys) && grid_of(64) <= INT_MAX) {
+        p.causal_waves = 4;
+        p.causal_kv_groups = D == 64 && kv_len >= kMinGroupKeys ? 2 : 1;
+    }
+}
 
 // ws_cap: most workspace a split prefill plan may ask for (it then takes
 // fewer KV partitions, or none); split decode plans ignore it, and
@@ -388,6 +437,7 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
             }
         }
     }
+    if (p.path == KF_PATH_PREFILL) plan_causal(p, q_len, kv_len, D, cus);
     if (p.path == KF_PATH_DECODE_SPLIT || p.path == KF_PATH_PREFILL_SPLIT) {
         const size_t parts = (size_t)p.n_splits * (size_t)rows_total;
         p.ws_o_off = 0;
@@ -432,8 +482,31 @@ void launch_prefill(const Plan& pl, const kf::AttnParams& prm, bool mask, hipStr
 
 // The prefill kernel of the plan (either prefill path).
 template <int D>
-hipError_t launch_prefill_kernel(const Plan& pl, const kf::AttnParams& prm, hipStream_t stream) {
-    const bool mask = prm.causal || prm.kv_lens;
+hipError_t launch_prefill_kernel(const Plan& plan, const kf::AttnParams& params, hipStream_t stream) {
+    const bool mask = params.causal || params.kv_lens;
+    Plan pl = plan;
+    kf::AttnParams prm = params;
+    if (prm.causal) {
+        // plan_causal's layouts.
+        const auto tiles = [&](int rows) {
+            pl.row_tiles = prm.row_tiles = (pl.R + rows - 1) / rows;
+            pl.grid = pl.n_groups * pl.row_tiles;
+        };
+        if (pl.causal_wide2) {
+            tiles(128);
+            pl.wide_row_tiles = pl.row_tiles;
+            pl.wide_grid = pl.grid;
+            pl.wide_kv_groups = 2;
+        } else if (pl.causal_groups == 2) {
+            tiles(128);
+            prm.causal_groups = 2;
+        } else if (pl.causal_waves > 0) {
+            pl.waves = pl.causal_waves;
+            pl.kv_groups = pl.causal_kv_groups;
+            pl.threads = 64 * pl.waves;
+            tiles(32 * pl.waves / pl.kv_groups);
+        }
+    }
     if constexpr (D >= 256) {
         if (pl.wide_row_tiles > 0) {
             kf::AttnParams pw = prm;
@@ -679,6 +752,9 @@ int run(const Plan& pl, kf::AttnParams prm, const void* Q, const void* K, const 
     prm.q_len = q_len;
     prm.heads_kv = H_kv;
     prm.xcds = pl.xcds;
+    prm.causal_sets = std::gcd(pl.n_groups, pl.xcds);
+    prm.causal_sets &= -prm.causal_sets;  // the power of two in it
+    prm.causal_per = pl.n_groups / prm.causal_sets;
 
     hipStream_t s = static_cast<hipStream_t>(stream);
     // Launch errors are read back with hipGetLastError(); clear whatever an
@@ -792,7 +868,12 @@ int kf_attn_kernel_names(int B, int q_len, int kv_len, int H_q, int H_kv, int D,
     if (prefill_path(pl.path)) {
         const bool causal = (flags & KF_ATTN_CAUSAL) != 0;
         const bool mask = causal || kv_lens;
-        if (pl.wide_row_tiles > 0 && causal && D < 256 && pl.wide_causal)
+        if (causal && pl.causal_wide2)
+            n = snprintf(tmp, sizeof(tmp), "kf_attn_prefill_wide_kernel<%d, true, 2, false>", D);
+        else if (causal && pl.causal_waves > 0)
+            n = snprintf(tmp, sizeof(tmp), "kf_attn_prefill_kernel<%d, true, %d, %d>", D, pl.causal_waves,
+                         pl.causal_kv_groups);
+        else if (pl.wide_row_tiles > 0 && causal && D < 256 && pl.wide_causal)
             n = snprintf(tmp, sizeof(tmp), "kf_attn_prefill_wide_kernel<%d, true, 1, true>", D);
         else if (pl.wide_row_tiles > 0 && (!causal || D >= 256))
             n = snprintf(tmp, sizeof(tmp), "kf_attn_prefill_wide_kernel<%d, %s, %d, false>", D,

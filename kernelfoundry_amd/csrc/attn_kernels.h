@@ -128,6 +128,8 @@ struct AttnParams {
     // XCDs of the device (8 on an MI355X in SPX mode, 1 per CPX partition):
     // the dispatcher deals workgroup ids round-robin over them.
     int xcds;
+    int causal_sets, causal_per;  // causal_place: sets of KV heads and XCDs, heads per set
+    int causal_groups;  // KV groups of the causal 8-wave kernel (1 or 2)
     // Ragged decode (kf_attn_decode_ragged_kernel).
     int batch;
     u32x4* ragged_heads;     // [B * H_kv] where a head's partials are
@@ -234,6 +236,50 @@ __device__ __forceinline__ void qi_range(int r0, int r1, int q_len, int& lo, int
     } else {
         lo = r0 % q_len;
         hi = r1 % q_len;
+    }
+}
+
+// Causal: the row tile that a KV head's k-th workgroup takes, longest first.
+// A tile's work grows with its rows' position inside their head, and the
+// dispatcher starts workgroups in order, so late, short tiles fill the CUs
+// that finish early.  Head hd owns the tiles that start in its rows, first(hd)
+// = ceil(hd q_len / rows) .. first(hd + 1) - 1: q_len / rows of them or one
+// more.  Workgroups go round the heads, each round one tile further from the
+// heads' ends; the heads with one more tile, their first, come last.  (Going
+// through the heads one after the other instead, as a q_len that is no
+// multiple of the tile did, S = 3000 at 32 / 8 heads, D = 128 ran 132 us.)
+__device__ __forceinline__ int causal_tile(int k, int row_tiles, int heads, int q_len, int rows) {
+    const int each = q_len / rows;
+    if (each == 0) return row_tiles - 1 - k;
+    auto first = [&](int hd) { return (hd * q_len + rows - 1) / rows; };  // hd q_len <= R, in range
+    const int j = k / heads;
+    if (j < each) return first(k - j * heads + 1) - 1 - j;
+    int left = k - each * heads;
+    for (int hd = 0; hd < heads; ++hd)
+        if (first(hd + 1) - first(hd) > each && left-- == 0) return first(hd);
+    return 0;  // not reached
+}
+
+// Causal, where a KV head's tiles run on several XCDs: workgroup id hw -> KV
+// head `grp` and its k-th row tile, longest first.  The heads and the XCDs
+// form `sets` sets of `per` heads each, as many as divide both (a power of
+// two); ids are dealt round-robin over the
+// XCDs, so set s = hw % sets owns XCDs s, s + sets, ... and exactly the ids of
+// its heads' tiles, which alternate between the set's XCDs, up to kCausalMix
+// heads side by side.  (xcd_remap's contiguous ranges would give one XCD a
+// head's long tiles and the next its short ones: MQA, 2048 queries at D = 64,
+// 4-wave workgroups 53.1 us so, 36.3 alternating.)
+constexpr int kCausalMix = 4;
+__device__ __forceinline__ void causal_place(int hw, int tiles, int sets, int per, int& grp, int& k) {
+    asm volatile("" ::: "memory");  // a branch of its own, not computed by every call
+    const int s = hw & (sets - 1), m = hw >> __builtin_ctz(sets);
+    if (per <= kCausalMix) {
+        k = m / per;
+        grp = s * per + m - k * per;
+    } else {
+        grp = m / tiles;
+        k = m - grp * tiles;
+        grp += s * per;
     }
 }
 
@@ -907,6 +953,19 @@ __device__ __forceinline__ void merge_kv_groups(const AttnParams& p, const RowSt
     }
 }
 
+// LDS of a prefill workgroup: three stage buffers (two: see PrefillCfg), for
+// 8-wave workgroups with KV groups the workgroup's query rows, copied once
+// (K's row layout) instead of KS times from memory, and the groups' row
+// statistics for their merge.
+template <int D, int NW, int KS> struct PrefillLds {
+    using Cfg = PrefillCfg<D, NW, KS>;
+    static constexpr int kBuf = KS * DmaStage<D, Cfg::kStageRows, Cfg::kRowWaves>::kStageBytes;
+    static constexpr int kBuf2 = Cfg::kBuffers == 3 ? kBuf : 16;
+    static constexpr bool kQLds = KS > 1 && NW == 8;
+    static constexpr int kQ = kQLds ? Cfg::kRows * D * 2 : 16;
+    static constexpr int kMl = KS > 1 ? 2 * NW * 64 : 1;  // floats
+};
+
 // kMask: causal masking and/or per-sequence key counts (p.causal,
 // p.kv_lens); without it every row sees keys [0, kv_len).
 //
@@ -921,8 +980,10 @@ __device__ __forceinline__ void merge_kv_groups(const AttnParams& p, const RowSt
 // it is a kernel of its own (kf_attn_prefill_parts_kernel), since its
 // registers would push the unsplit 4-wave kernel's past the architectural
 // VGPRs.
+// The LDS arrays are the kernel's (PrefillLds gives their sizes).
 template <int D, bool kMask, int NW, int KS, bool kParts>
-__device__ __forceinline__ void prefill_body(AttnParams p) {
+__device__ __forceinline__ void prefill_body(AttnParams p, char* buf0, char* buf1, char* buf2,
+                                             char* zero_pad, char* q_lds, float* merge_ml) {
     using Cfg = PrefillCfg<D, NW, KS>;
     constexpr int BC = Cfg::BC;
     constexpr int kNSB = BC / 32;                 // 32-row score blocks per stage
@@ -934,14 +995,7 @@ __device__ __forceinline__ void prefill_body(AttnParams p) {
     using SW = SwizzleRow<D>;
     constexpr int kNKK = D / 16;                  // MFMA k-steps over D
     constexpr int kNTD = (D < 32 ? 32 : D) / 32;  // 32-row O^T tiles
-    __shared__ __attribute__((aligned(1024))) char buf0[KS * S::kStageBytes];
-    __shared__ __attribute__((aligned(1024))) char buf1[KS * S::kStageBytes];
-    __shared__ __attribute__((aligned(1024))) char buf2[Cfg::kBuffers == 3 ? KS * S::kStageBytes : 16];
-    __shared__ __attribute__((aligned(16))) char zero_pad[16];  // D=16: V^T rows 16..31
-    // 8-wave workgroups with KV groups: the workgroup's query rows, copied
-    // once into LDS (K's row layout) instead of KS times from memory.
-    constexpr bool kQLds = KS > 1 && NW == 8;
-    __shared__ __attribute__((aligned(1024))) char q_lds[kQLds ? Cfg::kRows * D * 2 : 16];
+    constexpr bool kQLds = PrefillLds<D, NW, KS>::kQLds;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -961,23 +1015,15 @@ __device__ __forceinline__ void prefill_body(AttnParams p) {
     const bool split_out = kSplits && nsp > 1;
     const int split = blk % nsp;
     int rt = blk / nsp % p.row_tiles;
-    const int grp = blk / nsp / p.row_tiles;
+    int grp = blk / nsp / p.row_tiles;
     const int R = p.rows_per_group;
     const int kv_len = p.kv_len;
     const float c = p.scale_log2;
-    // Causal: a row tile's work grows with its position inside its head.
-    // Each XCD receives its groups' row tiles longest first, so late, short
-    // tiles fill the CUs that finish early: logical k -> position
-    // T - 1 - k / heads of head k % heads, T = row tiles per head (when
-    // tiles do not straddle heads; otherwise plain descending order).
     if (kMask && p.causal) {
-        const int q_len = p.q_len;
-        if (q_len % kPrefillRows == 0) {
-            const int T = q_len / kPrefillRows, heads = R / q_len;
-            rt = (rt % heads) * T + (T - 1 - rt / heads);
-        } else {
-            rt = p.row_tiles - 1 - rt;
-        }
+        // (One XCD per set: xcd_remap's ranges are the same.)
+        if (nsp == 1 && p.causal_sets != p.xcds)
+            causal_place(blockIdx.x, p.row_tiles, p.causal_sets, p.causal_per, grp, rt);
+        rt = causal_tile(rt, p.row_tiles, R / p.q_len, p.q_len, kPrefillRows);
     }
 
     // Keys this workgroup needs (blk_lim) and, per wave, the smallest row
@@ -1355,7 +1401,6 @@ __device__ __forceinline__ void prefill_body(AttnParams p) {
             char* bb = k / kSlotsPerBuf == 0 ? buf0 : (k / kSlotsPerBuf == 1 ? buf1 : buf2);
             return bb + (k % kSlotsPerBuf) * 1024;
         };
-        __shared__ float merge_ml[2 * KS * kRowWaves * 64];
         merge_kv_groups<D, KS, kRowWaves>(p, st, o, slot_base, merge_ml, wave, kgrp, lane, g,
                                           (size_t)grp * R + row,
                                           ((size_t)grp * nsp + split) * R + row, row < R);
@@ -1390,10 +1435,32 @@ __device__ __forceinline__ void prefill_body(AttnParams p) {
     }
 }
 
+// kTwo (the causal 8-wave kernel at D = 64 / 128): with p.causal_groups == 2
+// the workgroup takes 128 rows in two KV groups instead of 256 rows in one.  A
+// causal grid of one round of 256-row tiles lasts as long as its longest tile,
+// while the average row sees half its keys; twice as many tiles whose keys two
+// groups share halve the longest chain and fill the CUs longest first.  S =
+// 2048 at 32 / 8 heads: 67.4 -> 58 us (D = 128), 46.9 -> 39.5 (D = 64).
 template <int D, bool kMask, int NW = kPrefillMaxWaves<D>, int KS = 1>
 __global__ __launch_bounds__((PrefillCfg<D, NW, KS>::kThreads), (PrefillCfg<D, NW, KS>::kWavesPerEU))
 void kf_attn_prefill_kernel(AttnParams p) {
-    prefill_body<D, kMask, NW, KS, (D <= 128)>(p);
+    constexpr bool kTwo = kMask && NW == 8 && KS == 1 && (D == 64 || D == 128);
+    using L = PrefillLds<D, NW, KS>;
+    using L2 = PrefillLds<D, NW, kTwo ? 2 : KS>;
+    constexpr auto most = [](int a, int b) { return a > b ? a : b; };
+    __shared__ __attribute__((aligned(1024))) char buf0[most(L::kBuf, L2::kBuf)];
+    __shared__ __attribute__((aligned(1024))) char buf1[most(L::kBuf, L2::kBuf)];
+    __shared__ __attribute__((aligned(1024))) char buf2[most(L::kBuf2, L2::kBuf2)];
+    __shared__ __attribute__((aligned(16))) char zero_pad[16];  // D=16: V^T rows 16..31
+    __shared__ __attribute__((aligned(1024))) char q_lds[most(L::kQ, L2::kQ)];
+    __shared__ float merge_ml[most(L::kMl, L2::kMl)];
+    if constexpr (kTwo) {
+        if (p.causal_groups == 2) {
+            prefill_body<D, kMask, NW, 2, (D <= 128)>(p, buf0, buf1, buf2, zero_pad, q_lds, merge_ml);
+            return;
+        }
+    }
+    prefill_body<D, kMask, NW, KS, (D <= 128)>(p, buf0, buf1, buf2, zero_pad, q_lds, merge_ml);
 }
 
 // The split prefill at D = 256: the 4-wave kernel with KV partitions.
@@ -1401,7 +1468,11 @@ template <int D, bool kMask>
 __global__ __launch_bounds__((PrefillCfg<D, 4, 1>::kThreads), (PrefillCfg<D, 4, 1>::kWavesPerEU))
 void kf_attn_prefill_parts_kernel(AttnParams p) {
     static_assert(D == 256, "D <= 128 compiles the partitions into kf_attn_prefill_kernel");
-    prefill_body<D, kMask, 4, 1, true>(p);
+    using L = PrefillLds<D, 4, 1>;
+    __shared__ __attribute__((aligned(1024))) char buf0[L::kBuf];
+    __shared__ __attribute__((aligned(1024))) char buf1[L::kBuf];
+    __shared__ __attribute__((aligned(1024))) char buf2[L::kBuf2];
+    prefill_body<D, kMask, 4, 1, true>(p, buf0, buf1, buf2, nullptr, nullptr, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1508,19 +1579,14 @@ void kf_attn_prefill_wide_kernel(AttnParams p) {
     const int g = lane >> 5;
     const int blk = xcd_remap(blockIdx.x, gridDim.x, p.xcds);
     int rt = blk % p.row_tiles;
-    const int grp = blk / p.row_tiles;
+    int grp = blk / p.row_tiles;
     const int R = p.rows_per_group;
     const int kv_len = p.kv_len;
     const float c = p.scale_log2;
-    // Causal: row tiles longest first on every XCD (as kf_attn_prefill_kernel).
     if (causal) {
-        const int q_len = p.q_len;
-        if (q_len % kRows == 0) {
-            const int T = q_len / kRows, heads = R / q_len;
-            rt = (rt % heads) * T + (T - 1 - rt / heads);
-        } else {
-            rt = p.row_tiles - 1 - rt;
-        }
+        if (p.causal_sets != p.xcds)
+            causal_place(blockIdx.x, p.row_tiles, p.causal_sets, p.causal_per, grp, rt);
+        rt = causal_tile(rt, p.row_tiles, R / p.q_len, p.q_len, kRows);
     }
     // Keys this workgroup needs (blk_lim) and, per wave, the smallest row
     // limit (below it no masking is needed) and the largest (from it on
