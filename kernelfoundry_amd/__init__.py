@@ -258,14 +258,26 @@ def _out_flags(torch, out_dtype, return_lse):
 
 def _new(torch, shape, dtype, device, stream):
     """A new tensor written on ``stream``, allocated from ``stream``'s pool of
-    torch's caching allocator.  A block of that pool was last used by work on
+    torch's caching allocator (None: torch's current stream, without the
+    4 us that switching to it would take).  A block of that pool was last used by work on
     ``stream`` itself, so the launch that follows on ``stream`` is ordered
     after that work; a block taken from another stream's pool (torch's
     current one) could still be in use by a kernel queued there.  Freed, the
     tensor returns to ``stream``'s pool, so it is not reused before the
     launch on ``stream`` has finished with it."""
+    if stream is None:
+        return torch.empty(shape, dtype=dtype, device=device)
     with torch.cuda.stream(stream):
         return torch.empty(shape, dtype=dtype, device=device)
+
+
+def _raw_stream(torch, stream, device):
+    """The hipStream_t of ``stream``, or of torch's current one (read without
+    building the Stream object, 2 us, where torch has the call for it)."""
+    if stream is not None:
+        return stream.cuda_stream
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return raw(device.index) if raw else torch.cuda.current_stream(device).cuda_stream
 
 
 def _output(torch, out, shape, out_dtype, device, stream):
@@ -327,8 +339,6 @@ def attn_fwd(Q, K, V, out=None, *, return_stats=False, workspace=None, stream=No
     Bk, H_kv, kv_len, Dk = K.shape
     if Bk != B or Dk != D:
         raise ValueError("Q and K/V disagree on B or D")
-    if stream is None:
-        stream = torch.cuda.current_stream(Q.device)
     out = _output(torch, out, (B, H_q, q_len, D), out_dtype, Q.device, stream)
     Mi = Li = None
     if return_stats or return_lse:
@@ -355,7 +365,7 @@ def attn_fwd(Q, K, V, out=None, *, return_stats=False, workspace=None, stream=No
                          kv_lens.data_ptr() if kv_lens is not None else 0,
                          (KF_ATTN_CAUSAL if causal else 0) | flags,
                          workspace.data_ptr() if workspace is not None else 0,
-                         need, stream.cuda_stream)
+                         need, _raw_stream(torch, stream, Q.device))
     if st != KF_OK:
         msg = status_string(st)
         if st == KF_ERR_HIP:
@@ -397,8 +407,6 @@ def attn_decode_paged(Q, K_pages, V_pages, block_table, kv_lens, out=None, *, re
     if block_table.dim() != 2 or block_table.shape[0] != B or kv_lens.numel() != B:
         raise ValueError("block_table must be [B, max_pages_per_seq] and kv_lens [B]")
     max_pages = block_table.shape[1]
-    if stream is None:
-        stream = torch.cuda.current_stream(Q.device)
     out = _output(torch, out, (B, H_q, q_len, D), out_dtype, Q.device, stream)
     Mi = Li = None
     if return_stats or return_lse:
@@ -414,7 +422,7 @@ def attn_decode_paged(Q, K_pages, V_pages, block_table, kv_lens, out=None, *, re
                                B, q_len, H_q, H_kv, D, page_size, max_pages, num_pages,
                                (KF_ATTN_CAUSAL if causal else 0) | flags,
                                workspace.data_ptr() if workspace is not None else 0,
-                               need, stream.cuda_stream)
+                               need, _raw_stream(torch, stream, Q.device))
     if st != KF_OK:
         msg = status_string(st)
         if st == KF_ERR_HIP:
