@@ -67,6 +67,13 @@ constexpr int kMinSplitGroupKeys = 64;
 // Serial 32-key tiles per KV group a split prefill must save (measured at
 // 32 / 8 heads, D = 64 / 128: 4 saved tiles lose 3-22 %, 6 win 18-34 %).
 constexpr long long kMinSplitSavedTiles = 6;
+// Cost model of a split prefill's layouts, D = 128 (D = 64 tiles and partials
+// scale alike): a 32-key tile of a workgroup's KV groups, by 1, 2 and 4 groups
+// (per-wave stamps: 1.03, 1.21, 1.55 us), the partials written and read back,
+// the merge launch.
+constexpr double kSplitTileUs[3] = {1.03, 1.18, 1.55};
+constexpr double kSplitPartialBytesPerUs = 5e6;
+constexpr double kSplitMergeUs = 3.0;
 // Time of a 32-key tile of the 4-wave D = 256 prefill kernel (128 rows per
 // workgroup) relative to one of the wide kernel's KV groups (689 vs 487 us
 // for the whole S = 4096, 32 / 8 heads prefill).
@@ -194,6 +201,50 @@ size_t split_ws_bytes(size_t parts, int D) {
 }
 
 bool prefill_path(int path) { return path == KF_PATH_PREFILL || path == KF_PATH_PREFILL_SPLIT; }
+
+// A split of a prefill grid's keys into partitions (ns = 1: none).
+struct SplitChoice {
+    long long ns = 1, per = 0, row_tiles = 0;
+    int ks = 1;
+    double cost = 0.0;  // us: the tiles of one KV group and the partials' way to memory and back
+};
+
+// ns partitions for row_tiles tiles of ks KV groups each: as many as fit one
+// round of workgroups.
+SplitChoice split_prefill(const Plan& p, long long n_groups, long long R, long long kv_len, int D,
+                          long long rows_total, int ks, long long row_tiles, int cus, size_t ws_cap) {
+    SplitChoice none, c;
+    const long long grid = n_groups * row_tiles;
+    long long ns = cus / grid;
+    const long long by_keys = kv_len / ((long long)ks * kMinSplitGroupKeys);
+    if (ns > by_keys) ns = by_keys;
+    if (ns > kf::kMergeMaxSplits) ns = kf::kMergeMaxSplits;
+    while (ns > 1 && split_ws_bytes((size_t)ns * (size_t)rows_total, D) > ws_cap) --ns;
+    if (ns <= 1) return none;
+    // Partition length: whole tiles for every KV group.
+    const long long unit = 32LL * ks;
+    long long per = (kv_len + ns - 1) / ns;
+    per = (per + unit - 1) / unit * unit;
+    ns = (kv_len + per - 1) / per;
+    long long saved;
+    if (D == 256) {
+        const long long wunit = 32LL * (p.wide_row_tiles > 0 ? p.wide_kv_groups : 1);
+        const double chain = (double)((kv_len + wunit - 1) / wunit);
+        saved = (long long)(chain - kSplit256TileCost * (double)(per / 32));
+    } else {
+        saved = (kv_len + unit - 1) / unit - per / unit;  // tiles per KV group
+    }
+    const int cw = kf::merge_cols(D, (int)ns);
+    if (ns <= 1 || saved < kMinSplitSavedTiles || grid * ns > INT_MAX || rows_total * ((D / 4) / cw) > INT_MAX)
+        return none;
+    c.ns = ns;
+    c.per = per;
+    c.row_tiles = row_tiles;
+    c.ks = ks;
+    c.cost = kSplitTileUs[ks / 2] * (double)(per / unit) +
+             (double)ns * (double)rows_total * D * 8.0 / kSplitPartialBytesPerUs;
+    return c;
+}
 
 // The layout of an unsplit causal call where the unmasked one's is not the
 // best: a row sees kv_len - q_len / 2 keys on average against kv_len at most,
@@ -402,39 +453,38 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
         // split runs the 4-wave kernel, whose 32-key tile costs
         // kSplit256TileCost of a wide-kernel tile, against the wide kernel's
         // chain (halved by its two KV groups where it has them).
-        if ((p.wide_row_tiles == 0 || D == 256) && 2LL * p.grid <= cus) {
-            long long ns = cus / p.grid;
-            const long long by_keys = kv_len / ((long long)ks * kMinSplitGroupKeys);
-            if (ns > by_keys) ns = by_keys;
-            if (ns > kf::kMergeMaxSplits) ns = kf::kMergeMaxSplits;
-            while (ns > 1 && split_ws_bytes((size_t)ns * (size_t)rows_total, D) > ws_cap) --ns;
-            if (ns > 1) {
-                // Partition length: whole tiles for every KV group.
-                const long long unit = 32LL * ks;
-                long long per = (kv_len + ns - 1) / ns;
-                per = (per + unit - 1) / unit * unit;
-                ns = (kv_len + per - 1) / per;
-                long long saved;
-                if (D == 256) {
-                    const long long wunit = 32LL * (p.wide_row_tiles > 0 ? p.wide_kv_groups : 1);
-                    const double chain = (double)((kv_len + wunit - 1) / wunit);
-                    saved = (long long)(chain - kSplit256TileCost * (double)(per / 32));
-                } else {
-                    const long long tiles = ((long long)kv_len + unit - 1) / unit;  // per KV group, unsplit
-                    saved = tiles - per / unit;
-                }
-                const int cw = kf::merge_cols(D, (int)ns);
-                if (ns > 1 && saved >= kMinSplitSavedTiles && (long long)p.grid * ns <= INT_MAX && rows_total * ((D / 4) / cw) <= INT_MAX) {
-                    p.n_splits = (int)ns;
-                    p.kv_per_split = (int)per;
-                    p.grid = (int)((long long)p.grid * ns);
-                    p.merge_cw = cw;
-                    p.merge_per = kf::merge_per_lane(cw, p.n_splits);
-                    p.path = KF_PATH_PREFILL_SPLIT;
-                    p.wide_row_tiles = 0;  // D = 256: the 4-wave kernel
-                    p.wide_grid = 0;
+        // At D = 64 / 128 a split of the four-KV-group layout (64 rows per
+        // workgroup) is weighed against one of the two-group layout (128 rows,
+        // half as many row tiles, twice the partitions): its tiles cost less
+        // (kSplitTileUs), its partials twice as much.  us before -> now at 32 / 8
+        // heads, D = 128: 256 x 8192 60.1 -> 54.5, 256 x 16384 107 -> 91.6, 300 x
+        // 6000 67.4 -> 51.4, 512 x 16384 (unsplit before) 188 -> 167; D = 64
+        // 256 x 8192 40.5 -> 36.4.
+        const bool two = (D == 64 || D == 128) && nw == 8 && ks == 4 && R >= 128;
+        SplitChoice best;
+        if (p.wide_row_tiles == 0 || D == 256) {
+            if (2LL * p.grid <= cus)
+                best = split_prefill(p, n_groups, R, kv_len, D, rows_total, ks, p.row_tiles, cus, ws_cap);
+            if (two) {
+                const long long rt2 = (R + 127) / 128;
+                if (2 * n_groups * rt2 <= cus) {
+                    const SplitChoice c = split_prefill(p, n_groups, R, kv_len, D, rows_total, 2, rt2, cus, ws_cap);
+                    const double now = best.ns > 1 ? best.cost : kSplitTileUs[2] * (double)((kv_len + 127) / 128);
+                    if (c.ns > 1 && c.cost + (best.ns > 1 ? 0.0 : kSplitMergeUs) < now) best = c;
                 }
             }
+        }
+        if (best.ns > 1) {
+            p.kv_groups = best.ks;
+            p.row_tiles = (int)best.row_tiles;
+            p.n_splits = (int)best.ns;
+            p.kv_per_split = (int)best.per;
+            p.grid = (int)(n_groups * best.row_tiles * best.ns);
+            p.merge_cw = kf::merge_cols(D, p.n_splits);
+            p.merge_per = kf::merge_per_lane(p.merge_cw, p.n_splits);
+            p.path = KF_PATH_PREFILL_SPLIT;
+            p.wide_row_tiles = 0;  // D = 256: the 4-wave kernel
+            p.wide_grid = 0;
         }
     }
     if (p.path == KF_PATH_PREFILL) plan_causal(p, q_len, kv_len, D, cus);
