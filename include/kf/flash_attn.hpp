@@ -84,9 +84,21 @@ struct WorkspaceCache {
         return hipSuccess;
     }
 
+    // Whether `stream` is being captured (a capture on another stream that
+    // makes the question an error counts as no).
+    static bool capturing(hipStream_t stream) {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &status) == hipSuccess)
+            return status != hipStreamCaptureStatusNone;
+        (void)hipGetLastError();
+        return false;
+    }
+
     // A buffer of at least `need` bytes on the current device for `stream`
-    // (nullptr and 0 when need is 0).
-    hipError_t get(hipStream_t stream, size_t need, void** ptr, size_t* bytes) {
+    // (nullptr and 0 when need is 0).  Unless `grow_captured`, a stream under
+    // capture, where allocating is an error in most modes, gets the buffer as
+    // it is, smaller or none: many calls run with less than their best.
+    hipError_t get(hipStream_t stream, size_t need, void** ptr, size_t* bytes, bool grow_captured = true) {
         *ptr = nullptr;
         *bytes = 0;
         if (need == 0) return hipSuccess;
@@ -96,12 +108,14 @@ struct WorkspaceCache {
         Entry* en = nullptr;
         for (int i = 0; i < count && !en; ++i)
             if (entries[i].device == dev && entries[i].stream == stream) en = &entries[i];
+        const bool keep = !grow_captured && (!en || en->bytes < need) && capturing(stream);
+        if (!en && keep) return hipSuccess;
         if (!en) {
             if (count == kMaxEntries && (e = release(0)) != hipSuccess) return e;
             en = &entries[count++];
             *en = Entry{dev, stream, nullptr, 0};
         }
-        if (en->bytes < need) {
+        if (en->bytes < need && !keep) {
             if (en->ptr) {
                 // Kernels queued on this stream may still read the old buffer.
                 if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;
@@ -123,6 +137,23 @@ inline WorkspaceCache& thread_workspace() {
     return cache;
 }
 
+// launch(workspace, bytes) with `need` bytes; under capture first with what
+// the cache holds (KF_ERR_WORKSPACE launches nothing), so that a call that can
+// do without is captured without having run before.
+template <class Launch>
+hipError_t with_workspace(hipStream_t stream, size_t need, const Launch& launch) {
+    void* ws = nullptr;
+    size_t bytes = 0;
+    hipError_t e = thread_workspace().get(stream, need, &ws, &bytes, false);
+    if (e != hipSuccess) return e;
+    int st = launch(ws, bytes);
+    if (st == KF_ERR_WORKSPACE && bytes < need) {
+        if ((e = thread_workspace().get(stream, need, &ws, &bytes)) != hipSuccess) return e;
+        st = launch(ws, bytes);
+    }
+    return status_to_hip(st);
+}
+
 }  // namespace kf
 
 // Synchronous launcher with the reference signature (tests/test_flash_attn.cu:52-59).
@@ -141,13 +172,10 @@ inline hipError_t launch_flash_attn(const uint16_t* Q, const uint16_t* K, const 
     kf_attn_plan_t plan;
     int st = kf_attn_plan(B, q_len, kv_len, H_q, H_kv, D, &plan);
     if (st != KF_OK) return kf::status_to_hip(st);
-    void* ws = nullptr;
-    size_t ws_bytes = 0;
-    hipError_t e = kf::thread_workspace().get(stream, plan.workspace_bytes, &ws, &ws_bytes);
-    if (e != hipSuccess) return e;
-    st = kf_attn_fwd(Q, K, V, O, Mi, Li, B, q_len, kv_len, H_q, H_kv, D, ws, ws_bytes,
-                     static_cast<void*>(stream));
-    return kf::status_to_hip(st);
+    return kf::with_workspace(stream, plan.workspace_bytes, [&](void* ws, size_t ws_bytes) {
+        return kf_attn_fwd(Q, K, V, O, Mi, Li, B, q_len, kv_len, H_q, H_kv, D, ws, ws_bytes,
+                           static_cast<void*>(stream));
+    });
 }
 
 namespace kf {
@@ -164,13 +192,10 @@ inline hipError_t attn_fwd_ex(const uint16_t* Q, const uint16_t* K, const uint16
     if (st != KF_OK) return status_to_hip(st);
     const size_t need = kv_lens ? kf_attn_workspace_bytes_lens(B, q_len, kv_len, H_q, H_kv, D)
                                 : plan.workspace_bytes;
-    void* ws = nullptr;
-    size_t ws_bytes = 0;
-    hipError_t e = thread_workspace().get(stream, need, &ws, &ws_bytes);
-    if (e != hipSuccess) return e;
-    st = kf_attn_fwd_ex(Q, K, V, O, Mi, Li, B, q_len, kv_len, H_q, H_kv, D, kv_lens, flags,
-                        ws, ws_bytes, static_cast<void*>(stream));
-    return status_to_hip(st);
+    return with_workspace(stream, need, [&](void* ws, size_t ws_bytes) {
+        return kf_attn_fwd_ex(Q, K, V, O, Mi, Li, B, q_len, kv_len, H_q, H_kv, D, kv_lens, flags,
+                              ws, ws_bytes, static_cast<void*>(stream));
+    });
 }
 
 // kf_attn_decode_paged with the per-thread cached workspace.
@@ -182,15 +207,11 @@ inline hipError_t attn_decode_paged(const uint16_t* Q, const uint16_t* K_pages,
                                     float* Mi = nullptr, float* Li = nullptr) {
     const size_t need = kf_attn_decode_paged_workspace_bytes(B, q_len, H_q, H_kv, D, page_size,
                                                              max_pages_per_seq);
-    void* ws = nullptr;
-    size_t ws_bytes = 0;
-    hipError_t e = thread_workspace().get(stream, need, &ws, &ws_bytes);
-    if (e != hipSuccess) return e;
-    const int st = kf_attn_decode_paged(Q, K_pages, V_pages, block_table, kv_lens, O, Mi, Li, B,
-                                        q_len, H_q, H_kv, D, page_size, max_pages_per_seq,
-                                        num_pages, flags, ws, ws_bytes,
-                                        static_cast<void*>(stream));
-    return status_to_hip(st);
+    return with_workspace(stream, need, [&](void* ws, size_t ws_bytes) {
+        return kf_attn_decode_paged(Q, K_pages, V_pages, block_table, kv_lens, O, Mi, Li, B, q_len,
+                                    H_q, H_kv, D, page_size, max_pages_per_seq, num_pages, flags,
+                                    ws, ws_bytes, static_cast<void*>(stream));
+    });
 }
 
 }  // namespace kf
