@@ -199,7 +199,8 @@ int kf_attn_fwd_ex(const void* Q, const void* K, const void* V, void* O,
  * kf_attn_fwd_ex takes, in which case the results differ from its in the
  * last bits (both within the same tolerance of the exact result).  Likewise a
  * decode whose even sharing (kf_attn_workspace_bytes, or _lens) needs more than
- * the scratch runs by the plan's splits.
+ * the scratch runs by the plan's splits, and one whose plan needs no scratch
+ * takes none.
  * Every call on one device shares that device's array: calls that can run
  * concurrently on one device (two streams, two threads) race on it and must
  * be serialised by the caller; consecutive calls on one stream are safe.  The

@@ -8,6 +8,7 @@
 #include <atomic>
 #include <mutex>
 #include <climits>
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
@@ -74,6 +75,9 @@ constexpr long long kMinSplitSavedTiles = 6;
 constexpr double kSplitTileUs[3] = {1.03, 1.18, 1.55};
 constexpr double kSplitPartialBytesPerUs = 5e6;
 constexpr double kSplitMergeUs = 3.0;
+// Least saving for which the two-group layout is taken (32 queries against
+// 2000 keys at 32 / 8 heads, a predicted tie: 12.25 us in four, 12.76 in two).
+constexpr double kSplitTwoGain = 1.0;
 // Time of a 32-key tile of the 4-wave D = 256 prefill kernel (128 rows per
 // workgroup) relative to one of the wide kernel's KV groups (689 vs 487 us
 // for the whole S = 4096, 32 / 8 heads prefill).
@@ -188,6 +192,8 @@ struct Plan {
     size_t ragged_parts;  // its partials (two per worker) times rows
     size_t ragged_bytes;  // its workspace: the partials and the heads' table
     bool ragged_even;     // taken without key counts too
+    bool split_optional;  // split prefill that the four-group layout would run unsplit
+    int cus;            // compute units of the target device
     int xcds;           // XCDs of the target device (workgroup id remap)
 };
 
@@ -280,10 +286,14 @@ void plan_causal(Plan& p, int q_len, int kv_len, int D, int cus) {
     // 3000 113 -> 109, 3 x 1000 60.2 -> 54.2, 2 x 3000 205 -> 197, 4 x 1024
     // 69.6 -> 64.6, but 2 x 2048 98.4 -> 97.8 and 4096 165 -> 170; D = 64:
     // 3000 78.5 -> 71, 2 x 1000 31.3 -> 27.0.
+    // One round of 256-row tiles is cut so only with the KV groups (16 / 16
+    // heads, D = 64, 3 x 700 queries 18.1 us, 18.7 in 4-wave workgroups).
     const bool straddle = q_len % 256 != 0;
+    const int groups = D == 64 && kv_len >= kMinGroupKeys ? 2 : 1;
+    if (p.grid <= cus && groups == 1) return;
     if (avg_keys < (straddle ? kWideCausalMinKeys : kCausalShortKeys) && grid_of(64) <= INT_MAX) {
         p.causal_waves = 4;
-        p.causal_kv_groups = D == 64 && kv_len >= kMinGroupKeys ? 2 : 1;
+        p.causal_kv_groups = groups;
     }
 }
 
@@ -305,6 +315,7 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
         return KF_ERR_SIZE;
 
     Plan p{};
+    p.cus = dev.cus;
     p.xcds = dev.xcds;
     p.R = (int)R;
     p.n_groups = (int)n_groups;
@@ -462,19 +473,22 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
         // 256 x 8192 40.5 -> 36.4.
         const bool two = (D == 64 || D == 128) && nw == 8 && ks == 4 && R >= 128;
         SplitChoice best;
+        bool other = false;
         if (p.wide_row_tiles == 0 || D == 256) {
             if (2LL * p.grid <= cus)
                 best = split_prefill(p, n_groups, R, kv_len, D, rows_total, ks, p.row_tiles, cus, ws_cap);
+            other = best.ns > 1;
             if (two) {
                 const long long rt2 = (R + 127) / 128;
                 if (2 * n_groups * rt2 <= cus) {
                     const SplitChoice c = split_prefill(p, n_groups, R, kv_len, D, rows_total, 2, rt2, cus, ws_cap);
                     const double now = best.ns > 1 ? best.cost : kSplitTileUs[2] * (double)((kv_len + 127) / 128);
-                    if (c.ns > 1 && c.cost + (best.ns > 1 ? 0.0 : kSplitMergeUs) < now) best = c;
+                    if (c.ns > 1 && c.cost + (best.ns > 1 ? kSplitTwoGain : kSplitMergeUs) < now) best = c;
                 }
             }
         }
         if (best.ns > 1) {
+            p.split_optional = !other;
             p.kv_groups = best.ks;
             p.row_tiles = (int)best.row_tiles;
             p.n_splits = (int)best.ns;
@@ -556,6 +570,9 @@ hipError_t launch_prefill_kernel(const Plan& plan, const kf::AttnParams& params,
             pl.threads = 64 * pl.waves;
             tiles(32 * pl.waves / pl.kv_groups);
         }
+        // (The divisions of causal_place and causal_tile take up to 0.5 us of
+        // a small call: 4 x 150 queries, MQA at D = 128, 10.46 us without, 10.92 with.)
+        prm.causal_one_round = std::max(pl.grid, pl.wide_row_tiles > 0 ? pl.wide_grid : 0) <= pl.cus;
     }
     if constexpr (D >= 256) {
         if (pl.wide_row_tiles > 0) {
@@ -999,8 +1016,13 @@ int kf_attn_fwd_noalloc(const void* Q, const void* K, const void* V, void* O, fl
     st = check_args(flags, Q, K, V, O, kv_lens, nullptr);
     if (st != KF_OK) return st;
     if (pl.ws_bytes > kStaticScratchBytes) return KF_ERR_SCRATCH;
+    // A call that can do without scratch takes none: it may run next to another
+    // call on the device.  (The capacity plan then, where the ragged decode
+    // would want partials; a prefill that only the two-group layout splits
+    // runs unsplit.)
+    if (pl.split_optional) (void)make_plan(B, q_len, kv_len, H_q, H_kv, D, current_device_shape(), &pl, false, 0);
     void* ws = nullptr;
-    if (best_ws_bytes(pl, kv_lens != nullptr) > 0) {
+    if (pl.ws_bytes > 0) {
         hipError_t e = hipSuccess;
         ws = static_scratch(&e);
         if (!ws) return hip_fail(e);

@@ -129,6 +129,7 @@ struct AttnParams {
     // the dispatcher deals workgroup ids round-robin over them.
     int xcds;
     int causal_sets, causal_per;  // causal_place: sets of KV heads and XCDs, heads per set
+    int causal_one_round;  // a workgroup per CU at most: no order, the plain placement
     int causal_groups;  // KV groups of the causal 8-wave kernel (1 or 2)
     // Ragged decode (kf_attn_decode_ragged_kernel).
     int batch;
@@ -254,10 +255,10 @@ __device__ __forceinline__ int causal_tile(int k, int row_tiles, int heads, int 
     auto first = [&](int hd) { return (hd * q_len + rows - 1) / rows; };  // hd q_len <= R, in range
     const int j = k / heads;
     if (j < each) return first(k - j * heads + 1) - 1 - j;
-    int left = k - each * heads;
-    for (int hd = 0; hd < heads; ++hd)
-        if (first(hd + 1) - first(hd) > each && left-- == 0) return first(hd);
-    return 0;  // not reached
+    // The (left + 1)-th head with one more: its end is the first at which the
+    // remainders add up to more than `left` tiles.
+    const int left = k - each * heads;
+    return first(left * rows / (q_len - each * rows));
 }
 
 // Causal, where a KV head's tiles run on several XCDs: workgroup id hw -> KV
@@ -1021,9 +1022,11 @@ __device__ __forceinline__ void prefill_body(AttnParams p, char* buf0, char* buf
     const float c = p.scale_log2;
     if (kMask && p.causal) {
         // (One XCD per set: xcd_remap's ranges are the same.)
-        if (nsp == 1 && p.causal_sets != p.xcds)
-            causal_place(blockIdx.x, p.row_tiles, p.causal_sets, p.causal_per, grp, rt);
-        rt = causal_tile(rt, p.row_tiles, R / p.q_len, p.q_len, kPrefillRows);
+        if (__builtin_expect(!p.causal_one_round, 0)) {  // (out of the small calls' code)
+            if (nsp == 1 && p.causal_sets != p.xcds)
+                causal_place(blockIdx.x, p.row_tiles, p.causal_sets, p.causal_per, grp, rt);
+            rt = causal_tile(rt, p.row_tiles, R / p.q_len, p.q_len, kPrefillRows);
+        }
     }
 
     // Keys this workgroup needs (blk_lim) and, per wave, the smallest row
@@ -1584,9 +1587,11 @@ void kf_attn_prefill_wide_kernel(AttnParams p) {
     const int kv_len = p.kv_len;
     const float c = p.scale_log2;
     if (causal) {
-        if (p.causal_sets != p.xcds)
-            causal_place(blockIdx.x, p.row_tiles, p.causal_sets, p.causal_per, grp, rt);
-        rt = causal_tile(rt, p.row_tiles, R / p.q_len, p.q_len, kRows);
+        if (__builtin_expect(!p.causal_one_round, 0)) {  // (out of the small calls' code)
+            if (p.causal_sets != p.xcds)
+                causal_place(blockIdx.x, p.row_tiles, p.causal_sets, p.causal_per, grp, rt);
+            rt = causal_tile(rt, p.row_tiles, R / p.q_len, p.q_len, kRows);
+        }
     }
     // Keys this workgroup needs (blk_lim) and, per wave, the smallest row
     // limit (below it no masking is needed) and the largest (from it on
@@ -2569,13 +2574,13 @@ void kf_attn_decode_ragged_kernel(AttnParams p) {
             wait_vmcnt<kInstr>();  // V(t) has landed; K(t + 1) may be in flight
         else
             wait_vmcnt<0>();
-        if (kPaged && cs.bad) {
-            // V rows of an invalid page -> zeros, so that P = 0 meets finite
-            // values.  Rows past the keys repeat the last key's.
-            const int last = cs.k1 - cs.k0 - 1;
+        if (kPaged && (cs.bad || cs.k1 - cs.k0 < kDecodeStage)) {
+            // V rows past the keys (copies of the last key's) and of an
+            // invalid page -> zeros, so that P = 0 meets finite values.
             for (int i = lane; i < kDecodeStage * kChunks; i += 64) {
-                const int r = min(i / kChunks, last);
-                if (cs.bad >> (r >> 4) & 1) *reinterpret_cast<u32x4*>(vs + i * 16) = u32x4{0u, 0u, 0u, 0u};
+                const int r = i / kChunks;
+                if (r >= cs.k1 - cs.k0 || (cs.bad >> (r >> 4) & 1))
+                    *reinterpret_cast<u32x4*>(vs + i * 16) = u32x4{0u, 0u, 0u, 0u};
             }
             wave_lds_sync();
         }
@@ -2760,8 +2765,10 @@ void kf_attn_decode_ragged_kernel(AttnParams p) {
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int w = 0; w < NW; ++w)
-                if (mw[w] != -INFINITY) {
-                    const float wt = exp2_hw((mw[w] - m) * kLog2e);
+                if (w >= w0 && w < w1) {
+                    // Weight 0 for a row without a key here, whose sums are 0
+                    // (NaN if all of its scores were, which stays).
+                    const float wt = mw[w] == -INFINITY ? 0.f : exp2_hw((mw[w] - m) * kLog2e);
                     l += wt * lw[w];
                     acc += wt * ow[w];
                 }
@@ -2827,15 +2834,16 @@ void kf_attn_ragged_merge_kernel(AttnParams p) {
         float mx = m;
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) mx = fmaxf(mx, mv[u]);
-        if (mx == -INFINITY) continue;
-        const float keep = exp2_hw((m - mx) * kLog2e);
+        const bool none = mx == -INFINITY;            // weight 0 below keeps a NaN
+        const float keep = none ? 1.f : exp2_hw((m - mx) * kLog2e);
         acc *= keep;
         l *= keep;
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
-            const float w = k0 + u * kSL < ns ? exp2_hw((mv[u] - mx) * kLog2e) : 0.f;
-            l += w * lv[u];
-            acc += w * ov[u];
+            const bool in = k0 + u * kSL < ns;
+            const float w = in && !none ? exp2_hw((mv[u] - mx) * kLog2e) : 0.f;
+            l += in ? w * lv[u] : 0.f;
+            acc += in ? w * ov[u] : f32x4{0.f, 0.f, 0.f, 0.f};
         }
         m = mx;
     }

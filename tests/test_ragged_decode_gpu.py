@@ -167,3 +167,58 @@ def test_ragged_parity(case):
         assert np.abs(lse[full] - (Mr[full] + np.log(Lr[full]))).max() <= 1e-3
     # The same rows, rounded once.
     assert np.array_equal(O16.cpu().numpy(), O.astype(np.float16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,q,ps", [(16, 1, 16), (16, 4, 16), (12, 1, 0), (16, 4, 0)])
+def test_ragged_infinity_and_nan(B, q, ps):
+    """An infinity in a sequence's last V row, in a stage that other rows do
+    not fill, stays one and does not become NaN (0 times it; paged calls:
+    contiguous ones repeat that row), a query row of NaN gives NaN and no
+    other row does.  q = 1 and 4: partials straight to memory and by LDS."""
+    import torch
+    H_q, H_kv, cap, D = 32, 8, 4096, 128
+    print("case", B, q, ps, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(B + q)
+    normal = lambda *s: torch.randn(s, generator=gen, device="cuda", dtype=torch.float16)
+    lens = torch.tensor([1001 + 61 * b for b in range(B)], dtype=torch.int32, device="cuda")
+    Q = normal(B, H_q, q, D)
+    Q[1, 5, q - 1] = float("nan")
+    if ps:
+        need = cap // ps
+        K, V = normal(B * need, H_kv, ps, D), normal(B * need, H_kv, ps, D)
+        T = torch.arange(B * need, dtype=torch.int32, device="cuda").view(B, need)
+        last = int(lens[0]) - 1
+        V[T[0, last // ps].long(), :, last % ps, 7] = float("inf")
+        O = kf.attn_decode_paged(Q, K, V, T, lens)
+        assert torch.isposinf(O[0, :, :, 7]).all()
+        O[0, :, :, 7] = 0
+    else:
+        K, V = normal(B, H_kv, cap, D), normal(B, H_kv, cap, D)
+        O = kf.attn_fwd(Q, K, V, kv_lens=lens)
+    assert torch.isnan(O[1, 5, q - 1]).all()
+    O[1, 5, q - 1] = 0
+    assert torch.isfinite(O).all()
+
+
+@pytest.mark.gpu
+def test_noalloc_takes_no_scratch_where_the_plan_needs_none():
+    """kf_attn_fwd_noalloc shares its scratch between all calls on a device: a
+    call whose capacity plan is unsplit stays on that plan, so that it may run
+    next to another.  Bit for bit the call without a workspace."""
+    import torch
+    lib = kf.load_library()
+    B, q, cap, H_q, H_kv, D = shape = (32, 1, 4096, 32, 8, 128)
+    assert kf.workspace_bytes(*shape) == 0 < kf.workspace_bytes_lens(*shape)
+    print("case", shape, flush=True)
+    normal = lambda *s: torch.randn(s, device="cuda", dtype=torch.float16)
+    Q, K, V = normal(B, H_q, q, D), normal(B, H_kv, cap, D), normal(B, H_kv, cap, D)
+    lens = torch.from_numpy(_lens("mixed", B, cap, 5)).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+    A, C = torch.empty_like(Q, dtype=torch.float32), torch.empty_like(Q, dtype=torch.float32)
+    assert lib.kf_attn_fwd_noalloc(Q.data_ptr(), K.data_ptr(), V.data_ptr(), A.data_ptr(), None, None, *shape,
+                                   lens.data_ptr(), 0, stream) == kf.KF_OK
+    assert kf.attn_fwd_ex_ptr(Q.data_ptr(), K.data_ptr(), V.data_ptr(), C.data_ptr(), 0, 0, *shape,
+                              kv_lens=lens.data_ptr(), stream=stream) == kf.KF_OK
+    torch.cuda.synchronize()
+    assert torch.equal(A, C)
