@@ -25,6 +25,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <vector>
 
 #include "kf/attn.h"
 
@@ -49,20 +50,42 @@ inline hipError_t status_to_hip(int st) {
 // Entries are keyed by the stream handle: a stream destroyed while its
 // launches still run may hand its handle to a new stream, which would then
 // share the buffer, so synchronise a stream before destroying it.
+//
+// A graph captured from these launchers holds the buffer's address.  Such a
+// buffer is not freed when its entry grows or is released, only with the
+// thread's cache, so a graph may be replayed until the thread that captured
+// it ends.  Until its entry grows the graph shares the buffer with later
+// launches on the captured stream: replay it there, or ordered with them.
 struct WorkspaceCache {
     struct Entry {
         int device;
         hipStream_t stream;
         void* ptr;
         size_t bytes;
+        bool captured;  // ptr has been handed to a stream under capture
     };
     static constexpr int kMaxEntries = 16;
     Entry entries[kMaxEntries] = {};
     int count = 0;
+    std::vector<void*> retired;  // captured buffers that no entry holds any more
 
     ~WorkspaceCache() {
         for (int i = 0; i < count; ++i)
             if (entries[i].ptr) (void)hipFree(entries[i].ptr);
+        for (void* ptr : retired) (void)hipFree(ptr);
+    }
+
+    // Entry i gives up its buffer, which no kernel queued outside a graph
+    // uses any more: freed, or kept for the graphs that hold it.
+    hipError_t drop(int i) {
+        Entry& en = entries[i];
+        void* ptr = en.ptr;
+        const bool keep = en.captured;
+        if (keep) retired.push_back(ptr);
+        en.ptr = nullptr;
+        en.bytes = 0;
+        en.captured = false;
+        return keep ? hipSuccess : hipFree(ptr);
     }
 
     // Drop entry i: its kernels may still run, so its device is drained
@@ -74,7 +97,7 @@ struct WorkspaceCache {
         if (entries[i].ptr) {
             if ((e = hipSetDevice(entries[i].device)) != hipSuccess) return e;
             e = hipDeviceSynchronize();
-            if (e == hipSuccess) e = hipFree(entries[i].ptr);
+            if (e == hipSuccess) e = drop(i);
             const hipError_t e2 = hipSetDevice(cur);
             if (e != hipSuccess) return e;
             if (e2 != hipSuccess) return e2;
@@ -108,24 +131,24 @@ struct WorkspaceCache {
         Entry* en = nullptr;
         for (int i = 0; i < count && !en; ++i)
             if (entries[i].device == dev && entries[i].stream == stream) en = &entries[i];
-        const bool keep = !grow_captured && (!en || en->bytes < need) && capturing(stream);
+        const bool captured = capturing(stream);
+        const bool keep = !grow_captured && (!en || en->bytes < need) && captured;
         if (!en && keep) return hipSuccess;
         if (!en) {
             if (count == kMaxEntries && (e = release(0)) != hipSuccess) return e;
             en = &entries[count++];
-            *en = Entry{dev, stream, nullptr, 0};
+            *en = Entry{dev, stream, nullptr, 0, false};
         }
         if (en->bytes < need && !keep) {
             if (en->ptr) {
                 // Kernels queued on this stream may still read the old buffer.
                 if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;
-                (void)hipFree(en->ptr);
-                en->ptr = nullptr;
-                en->bytes = 0;
+                (void)drop(static_cast<int>(en - entries));
             }
             if ((e = hipMalloc(&en->ptr, need)) != hipSuccess) return e;
             en->bytes = need;
         }
+        en->captured = en->captured || (captured && en->ptr);
         *ptr = en->ptr;
         *bytes = en->bytes;
         return hipSuccess;

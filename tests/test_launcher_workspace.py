@@ -29,7 +29,10 @@ inline hipError_t busy() { return g_capturing ? hipErrorStreamCaptureUnsupported
 inline hipError_t hipDeviceSynchronize() { return busy(); }
 inline hipError_t hipStreamSynchronize(hipStream_t) { return busy(); }
 inline hipError_t hipGetLastError() { return hipSuccess; }
-inline hipError_t hipFree(void* p) { free(p); return hipSuccess; }
+inline int g_frees = 0;
+inline void* g_freed[1000];
+// (Kept, so that no later buffer has a freed one's address.)
+inline hipError_t hipFree(void* p) { g_freed[g_frees++] = p; return hipSuccess; }
 inline hipError_t hipMalloc(void** p, size_t n) {
     if (g_capturing) return hipErrorStreamCaptureUnsupported;
     ++g_mallocs;
@@ -47,6 +50,7 @@ MAIN = r"""
 #include <cstdio>
 // The call needs `least` bytes and runs best with `best`.
 static size_t least, best, got;
+static void* got_ws;
 extern "C" {
 int kf_last_hip_error(void) { return 0; }
 int kf_launch_flash_attn(const uint16_t*, const uint16_t*, const uint16_t*, float*, int, int, int, int, int,
@@ -57,6 +61,7 @@ size_t kf_attn_decode_paged_workspace_bytes(int, int, int, int, int, int, int) {
 static int take(void* ws, size_t n) {
     if (least && (!ws || n < least)) return KF_ERR_WORKSPACE;
     got = ws ? n : 0;
+    got_ws = ws;
     return KF_OK;
 }
 int kf_attn_fwd(const void*, const void*, const void*, float*, float*, float*, int, int, int, int, int, int,
@@ -77,6 +82,9 @@ static hipError_t call(int i, long stream, size_t need, size_t want) {
     return kf::attn_decode_paged(nullptr, nullptr, nullptr, nullptr, &lens, nullptr, 1, 1, 1, 1, 16, 16, 1, 1, 0, s);
 }
 #define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
+"""
+
+UNDER_CAPTURE = r"""
 int main() {
     for (int i = 0; i < 3; ++i) {
         const long s = 8 * i;
@@ -104,11 +112,56 @@ int main() {
 """
 
 
+# A buffer handed out under capture belongs to the graph: what later calls free
+# (on growth, on release of the entry) never includes it.
+CAPTURED_BUFFERS = r"""
+static bool freed(void* p) {
+    for (int i = 0; i < g_frees; ++i)
+        if (g_freed[i] == p) return true;
+    return false;
+}
+int main() {
+    for (int i = 0; i < 3; ++i) {
+        const long s = 8 * i;
+        // Captured with less than its best, then an eager call of the same shape.
+        CHECK(call(i, s + 1, 256, 256) == hipSuccess);
+        void* const small = got_ws;
+        g_capturing = true;
+        CHECK(call(i, s + 1, 256, 512) == hipSuccess && got_ws == small);
+        g_capturing = false;
+        CHECK(call(i, s + 1, 256, 512) == hipSuccess && got == 512 && got_ws != small && !freed(small));
+        // Captured at its best, then a larger call.
+        void* const best_ws = got_ws;
+        g_capturing = true;
+        CHECK(call(i, s + 1, 256, 512) == hipSuccess && got_ws == best_ws);
+        g_capturing = false;
+        CHECK(call(i, s + 1, 1024, 1024) == hipSuccess && got == 1024 && !freed(best_ws));
+        // The buffer that followed was not captured: it goes as it grows.
+        void* const eager = got_ws;
+        CHECK(call(i, s + 1, 2048, 2048) == hipSuccess && freed(eager));
+    }
+    // Every entry released: the captured buffer stays, the others go.
+    CHECK(call(1, 99, 16, 16) == hipSuccess);
+    void* const kept = got_ws;
+    g_capturing = true;
+    CHECK(call(1, 99, 16, 16) == hipSuccess && got_ws == kept);
+    g_capturing = false;
+    CHECK(call(1, 100, 16, 16) == hipSuccess);
+    void* const gone = got_ws;
+    for (long s = 101; s < 140; ++s) CHECK(call(1, s, 16, 16) == hipSuccess);
+    CHECK(!freed(kept) && freed(gone));
+    std::printf("ok\n");
+    return 0;
+}
+"""
+
+
 @pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
-def test_launchers_under_capture(tmp_path):
+@pytest.mark.parametrize("body", [UNDER_CAPTURE, CAPTURED_BUFFERS], ids=["under_capture", "captured_buffers"])
+def test_launchers_under_capture(tmp_path, body):
     (tmp_path / "hip").mkdir()
     (tmp_path / "hip" / "hip_runtime.h").write_text(HIP)
-    (tmp_path / "main.cpp").write_text(MAIN)
+    (tmp_path / "main.cpp").write_text(MAIN + body)
     exe = tmp_path / "main"
     subprocess.run(["g++", "-std=c++17", "-O1", f"-I{tmp_path}", f"-I{INCLUDE}", str(tmp_path / "main.cpp"),
                     "-o", str(exe)], check=True, capture_output=True, timeout=120)
