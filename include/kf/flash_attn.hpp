@@ -67,6 +67,7 @@ struct WorkspaceCache {
     static constexpr int kMaxEntries = 16;
     Entry entries[kMaxEntries] = {};
     int count = 0;
+    bool out_of_memory = false;  // the last get() failed because no memory was left
     std::vector<void*> retired;  // captured buffers that no entry holds any more
 
     ~WorkspaceCache() {
@@ -124,6 +125,7 @@ struct WorkspaceCache {
     hipError_t get(hipStream_t stream, size_t need, void** ptr, size_t* bytes, bool grow_captured = true) {
         *ptr = nullptr;
         *bytes = 0;
+        out_of_memory = false;
         if (need == 0) return hipSuccess;
         int dev = 0;
         hipError_t e = hipGetDevice(&dev);
@@ -145,7 +147,12 @@ struct WorkspaceCache {
                 if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;
                 (void)drop(static_cast<int>(en - entries));
             }
-            if ((e = hipMalloc(&en->ptr, need)) != hipSuccess) return e;
+            if ((e = hipMalloc(&en->ptr, need)) != hipSuccess) {
+                en->ptr = nullptr;
+                out_of_memory = !captured;
+                (void)hipGetLastError();
+                return e;
+            }
             en->bytes = need;
         }
         en->captured = en->captured || (captured && en->ptr);
@@ -160,18 +167,35 @@ inline WorkspaceCache& thread_workspace() {
     return cache;
 }
 
-// launch(workspace, bytes) with `need` bytes; under capture first with what
-// the cache holds (KF_ERR_WORKSPACE launches nothing), so that a call that can
-// do without is captured without having run before.
-template <class Launch>
-hipError_t with_workspace(hipStream_t stream, size_t need, const Launch& launch) {
+// The split partials of `rows` query rows by the plan, without which a split
+// decode does not run (any other call runs without a workspace).
+inline size_t plan_partial_bytes(const kf_attn_plan_t& plan, size_t rows, int D) {
+    if (plan.path != KF_PATH_DECODE_SPLIT) return 0;
+    const auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+    const size_t parts = static_cast<size_t>(plan.num_splits) * rows;
+    return up(parts * static_cast<size_t>(D) * sizeof(float)) + 2 * up(parts * sizeof(float));
+}
+
+// launch(workspace, bytes) with `need` bytes.  (KF_ERR_WORKSPACE launches
+// nothing.)  Under capture first with what the cache holds, so that a call
+// that can do without is captured without having run before.  Where `need`
+// bytes are not to be had, without a workspace or with the least() bytes that
+// the call cannot do without.
+template <class Least, class Launch>
+hipError_t with_workspace(hipStream_t stream, size_t need, const Least& least, const Launch& launch) {
+    WorkspaceCache& cache = thread_workspace();
     void* ws = nullptr;
     size_t bytes = 0;
-    hipError_t e = thread_workspace().get(stream, need, &ws, &bytes, false);
-    if (e != hipSuccess) return e;
+    hipError_t e = cache.get(stream, need, &ws, &bytes, false);
+    if (e != hipSuccess && !cache.out_of_memory) return e;
     int st = launch(ws, bytes);
     if (st == KF_ERR_WORKSPACE && bytes < need) {
-        if ((e = thread_workspace().get(stream, need, &ws, &bytes)) != hipSuccess) return e;
+        size_t ask = need;
+        if (e != hipSuccess) {
+            ask = least();
+            if (ask == 0 || ask >= need) return e;
+        }
+        if ((e = cache.get(stream, ask, &ws, &bytes)) != hipSuccess) return e;
         st = launch(ws, bytes);
     }
     return status_to_hip(st);
@@ -192,10 +216,11 @@ inline hipError_t launch_flash_attn(const uint16_t* Q, const uint16_t* K, const 
                                     float* O, int B, int q_len, int kv_len, int H_q, int H_kv,
                                     int D, hipStream_t stream, float* Mi = nullptr,
                                     float* Li = nullptr) {
-    kf_attn_plan_t plan;
+    kf_attn_plan_t plan{};
     int st = kf_attn_plan(B, q_len, kv_len, H_q, H_kv, D, &plan);
     if (st != KF_OK) return kf::status_to_hip(st);
-    return kf::with_workspace(stream, plan.workspace_bytes, [&](void* ws, size_t ws_bytes) {
+    const auto least = [&] { return kf::plan_partial_bytes(plan, size_t(B) * H_q * q_len, D); };
+    return kf::with_workspace(stream, plan.workspace_bytes, least, [&](void* ws, size_t ws_bytes) {
         return kf_attn_fwd(Q, K, V, O, Mi, Li, B, q_len, kv_len, H_q, H_kv, D, ws, ws_bytes,
                            static_cast<void*>(stream));
     });
@@ -210,12 +235,13 @@ inline hipError_t attn_fwd_ex(const uint16_t* Q, const uint16_t* K, const uint16
                               int B, int q_len, int kv_len, int H_q, int H_kv, int D,
                               const int* kv_lens, int flags, hipStream_t stream,
                               float* Mi = nullptr, float* Li = nullptr) {
-    kf_attn_plan_t plan;
+    kf_attn_plan_t plan{};
     int st = kf_attn_plan(B, q_len, kv_len, H_q, H_kv, D, &plan);
     if (st != KF_OK) return status_to_hip(st);
+    const auto least = [&] { return plan_partial_bytes(plan, size_t(B) * H_q * q_len, D); };
     const size_t need = kv_lens ? kf_attn_workspace_bytes_lens(B, q_len, kv_len, H_q, H_kv, D)
                                 : plan.workspace_bytes;
-    return with_workspace(stream, need, [&](void* ws, size_t ws_bytes) {
+    return with_workspace(stream, need, least, [&](void* ws, size_t ws_bytes) {
         return kf_attn_fwd_ex(Q, K, V, O, Mi, Li, B, q_len, kv_len, H_q, H_kv, D, kv_lens, flags,
                               ws, ws_bytes, static_cast<void*>(stream));
     });
@@ -230,7 +256,13 @@ inline hipError_t attn_decode_paged(const uint16_t* Q, const uint16_t* K_pages,
                                     float* Mi = nullptr, float* Li = nullptr) {
     const size_t need = kf_attn_decode_paged_workspace_bytes(B, q_len, H_q, H_kv, D, page_size,
                                                              max_pages_per_seq);
-    return with_workspace(stream, need, [&](void* ws, size_t ws_bytes) {
+    const auto least = [&]() -> size_t {
+        kf_attn_plan_t plan{};
+        const int cap = page_size * max_pages_per_seq;  // need > 0: a valid geometry
+        if (kf_attn_plan(B, q_len, cap, H_q, H_kv, D, &plan) != KF_OK) return 0;
+        return plan_partial_bytes(plan, size_t(B) * H_q * q_len, D);
+    };
+    return with_workspace(stream, need, least, [&](void* ws, size_t ws_bytes) {
         return kf_attn_decode_paged(Q, K_pages, V_pages, block_table, kv_lens, O, Mi, Li, B, q_len,
                                     H_q, H_kv, D, page_size, max_pages_per_seq, num_pages, flags,
                                     ws, ws_bytes, static_cast<void*>(stream));

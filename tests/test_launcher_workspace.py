@@ -19,10 +19,11 @@ HIP = r"""
 #include <cstdint>
 #include <cstdlib>
 typedef struct S* hipStream_t;
-enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorStreamCaptureUnsupported = 900 };
+enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorStreamCaptureUnsupported = 900 };
 enum hipStreamCaptureStatus { hipStreamCaptureStatusNone, hipStreamCaptureStatusActive };
 inline bool g_capturing = false;
 inline int g_mallocs = 0;
+inline size_t g_memory = SIZE_MAX;   // the largest allocation that succeeds
 inline hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t busy() { return g_capturing ? hipErrorStreamCaptureUnsupported : hipSuccess; }
@@ -35,6 +36,7 @@ inline void* g_freed[1000];
 inline hipError_t hipFree(void* p) { g_freed[g_frees++] = p; return hipSuccess; }
 inline hipError_t hipMalloc(void** p, size_t n) {
     if (g_capturing) return hipErrorStreamCaptureUnsupported;
+    if (n > g_memory) return hipErrorOutOfMemory;
     ++g_mallocs;
     *p = malloc(n);
     return hipSuccess;
@@ -55,7 +57,12 @@ extern "C" {
 int kf_last_hip_error(void) { return 0; }
 int kf_launch_flash_attn(const uint16_t*, const uint16_t*, const uint16_t*, float*, int, int, int, int, int,
                          void*) { return 0; }
-int kf_attn_plan(int, int, int, int, int, int, kf_attn_plan_t* p) { p->workspace_bytes = best; return KF_OK; }
+int kf_attn_plan(int, int, int, int, int, int, kf_attn_plan_t* p) {
+    p->workspace_bytes = best;
+    p->path = least ? KF_PATH_DECODE_SPLIT : KF_PATH_DECODE;
+    p->num_splits = 4;
+    return KF_OK;
+}
 size_t kf_attn_workspace_bytes_lens(int, int, int, int, int, int) { return best; }
 size_t kf_attn_decode_paged_workspace_bytes(int, int, int, int, int, int, int) { return best; }
 static int take(void* ws, size_t n) {
@@ -155,13 +162,37 @@ int main() {
 }
 """
 
+# No memory for a call's best: it runs without a workspace, or with the partials
+# of its plan (4 splits of one row at D = 16: 256 bytes, and 256 for each of the
+# two statistics).
+OUT_OF_MEMORY = r"""
+int main() {
+    for (int i = 0; i < 3; ++i) {
+        const long s = 8 * i;
+        g_memory = 1000;
+        CHECK(call(i, s + 1, 0, 4096) == hipSuccess && got == 0);
+        CHECK(call(i, s + 1, 768, 4096) == hipSuccess && got == 768);
+        CHECK(call(i, s + 1, 768, 4096) == hipSuccess && got == 768);
+        CHECK(call(i, s + 1, 768, 768) == hipSuccess && got == 768);
+        g_memory = 700;
+        CHECK(call(i, s + 2, 768, 4096) == hipErrorOutOfMemory);
+        CHECK(call(i, s + 2, 768, 768) == hipErrorOutOfMemory);
+        g_memory = SIZE_MAX;
+        CHECK(call(i, s + 2, 768, 4096) == hipSuccess && got == 4096);
+    }
+    std::printf("ok\n");
+    return 0;
+}
+"""
+BODIES = {"under_capture": UNDER_CAPTURE, "captured_buffers": CAPTURED_BUFFERS, "out_of_memory": OUT_OF_MEMORY}
+
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
-@pytest.mark.parametrize("body", [UNDER_CAPTURE, CAPTURED_BUFFERS], ids=["under_capture", "captured_buffers"])
+@pytest.mark.parametrize("body", list(BODIES))
 def test_launchers_under_capture(tmp_path, body):
     (tmp_path / "hip").mkdir()
     (tmp_path / "hip" / "hip_runtime.h").write_text(HIP)
-    (tmp_path / "main.cpp").write_text(MAIN + body)
+    (tmp_path / "main.cpp").write_text(MAIN + BODIES[body])
     exe = tmp_path / "main"
     subprocess.run(["g++", "-std=c++17", "-O1", f"-I{tmp_path}", f"-I{INCLUDE}", str(tmp_path / "main.cpp"),
                     "-o", str(exe)], check=True, capture_output=True, timeout=120)
