@@ -1057,8 +1057,17 @@ __device__ __forceinline__ void prefill_body(AttnParams p, char* buf0, char* buf
     // KV group kgrp covers [kv_base, kv_end) of them in tiles 0 .. ntiles - 1
     // (the same count for every group); row limits below are relative to
     // kv_base.
-    const int s0 = split * p.kv_per_split;
-    if (split_out) blk_lim = min(blk_lim, s0 + p.kv_per_split);
+    int per = p.kv_per_split;
+    if constexpr (kMask && kSplits && KS == 2) {
+        // Two KV groups: the partitions share the keys that the sequence has,
+        // not its capacity, which would leave partitions of a short one without
+        // keys and give the others' to half the groups of the four-group layout
+        // (243 queries, 32 / 8 heads, D = 128, capacity 9605, 1200 keys: 29.2 us
+        // by capacity, 23.5 in four groups, 18.9 so; 300 keys 17.2, 14.6, 14.7).
+        if (split_out && p.kv_lens) per = ((kvb + nsp - 1) / nsp + 32 * KS - 1) / (32 * KS) * (32 * KS);
+    }
+    const int s0 = split * per;
+    if (split_out) blk_lim = min(blk_lim, s0 + per);
     const int ntiles_wg = max(blk_lim - s0 + BC - 1, 0) / BC;
     const int ntiles = KS == 1 ? ntiles_wg : (ntiles_wg + KS - 1) / KS;  // 32-row tiles
     const int nstages = (ntiles * BC + SR - 1) / SR;                     // LDS stages

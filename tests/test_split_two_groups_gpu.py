@@ -14,6 +14,8 @@ CASES = [
     (1, 32, 4, 500, 4095, 128, True, None),              # unsplit by the four-group layout
     (2, 16, 4, 256, 5000, 64, True, [5000, 130]),        # partitions past 130 keys, rows without any
     (2, 16, 4, 256, 5000, 64, False, [0, 4999]),         # an empty sequence
+    (1, 32, 8, 243, 9605, 128, True, [1300]),            # keys shared by all partitions
+    (3, 8, 2, 256, 9000, 128, False, [1, 65, 1111]),     # partitions of one tile, and without keys
 ]
 
 
@@ -60,3 +62,25 @@ def test_smaller_workspaces_agree():
                                 workspace_bytes=n, stream=torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
         assert st == kf.KF_OK and (O - ref).abs().max().item() <= 2e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+def test_partitions_share_a_short_sequences_keys(D):
+    """Every partition of a sequence that fills an eighth of its capacity has
+    keys (a finite row maximum in its partials), one that fills all of it gives
+    the bits of the call without key counts."""
+    import torch
+    B, H_q, H_kv, q, kv = 1, 32, 8, 256, 8192
+    print("case short sequence", D, flush=True)
+    p = kf.plan(B, q, kv, H_q, H_kv, D)
+    assert p.path == "prefill_split" and "8, 2>" in kf.kernel_names(B, q, kv, H_q, H_kv, D, masked=True)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    Q, K, V = (torch.randn((B, h, n, D), generator=g, dtype=torch.float16, device="cuda")
+               for h, n in ((H_q, q), (H_kv, kv), (H_kv, kv)))
+    ws = torch.zeros(p.workspace_bytes // 4, dtype=torch.float32, device="cuda")
+    lens = lambda n: torch.tensor([n], dtype=torch.int32, device="cuda")
+    kf.attn_fwd(Q, K, V, kv_lens=lens(kv // 8), workspace=ws)
+    parts = p.num_splits * B * H_q * q           # O partials, then the row maxima
+    assert torch.isfinite(ws[parts * D:parts * (D + 1)]).all()
+    assert torch.equal(kf.attn_fwd(Q, K, V, kv_lens=lens(kv)), kf.attn_fwd(Q, K, V, kv_lens=None))
