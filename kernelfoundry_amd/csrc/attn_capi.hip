@@ -68,16 +68,22 @@ constexpr int kMinSplitGroupKeys = 64;
 // Serial 32-key tiles per KV group a split prefill must save (measured at
 // 32 / 8 heads, D = 64 / 128: 4 saved tiles lose 3-22 %, 6 win 18-34 %).
 constexpr long long kMinSplitSavedTiles = 6;
-// Cost model of a split prefill's layouts, D = 128 (D = 64 tiles and partials
-// scale alike): a 32-key tile of a workgroup's KV groups, by 1, 2 and 4 groups
-// (per-wave stamps: 1.03, 1.21, 1.55 us), the partials written and read back,
-// the merge launch.
-constexpr double kSplitTileUs[3] = {1.03, 1.18, 1.55};
+// Cost model of a split prefill's layouts: a 32-key tile of a workgroup's KV
+// groups, by 1, 2 and 4 groups (D = 128 from per-wave stamps, rounded; D = 64
+// fitted to 480 shapes run in both layouts), the partials written and read
+// back, the merge launch, and the least saving for which the two-group layout
+// is taken (32 queries against 2000 keys at 32 / 8 heads, D = 128, a predicted
+// tie: 12.25 us in four, 12.76 in two).  An unsplit four-group call at D = 64,
+// whose tiles a workgroup's fixed part hides better, also waits for K and V
+// from memory.  At D = 64 with D = 128's tile costs, 256 x 1024 at 32 / 8 heads
+// went from 11.8 us to 13.4, 64 x 2048 for 6 sequences from 19.3 to 22.2.
+struct SplitCosts {
+    double tile[3], unsplit_tile, unsplit_kv_mb, merge, two_gain;
+};
+constexpr SplitCosts kSplitCosts64 = {{0.0, 0.75, 1.0}, 0.93, 0.05, 3.5, 0.7};
+constexpr SplitCosts kSplitCosts128 = {{1.03, 1.18, 1.55}, 1.55, 0.0, 3.0, 1.0};
+constexpr const SplitCosts& split_costs(int D) { return D == 64 ? kSplitCosts64 : kSplitCosts128; }
 constexpr double kSplitPartialBytesPerUs = 5e6;
-constexpr double kSplitMergeUs = 3.0;
-// Least saving for which the two-group layout is taken (32 queries against
-// 2000 keys at 32 / 8 heads, a predicted tie: 12.25 us in four, 12.76 in two).
-constexpr double kSplitTwoGain = 1.0;
 // Time of a 32-key tile of the 4-wave D = 256 prefill kernel (128 rows per
 // workgroup) relative to one of the wide kernel's KV groups (689 vs 487 us
 // for the whole S = 4096, 32 / 8 heads prefill).
@@ -247,7 +253,7 @@ SplitChoice split_prefill(const Plan& p, long long n_groups, long long R, long l
     c.per = per;
     c.row_tiles = row_tiles;
     c.ks = ks;
-    c.cost = kSplitTileUs[ks / 2] * (double)(per / unit) +
+    c.cost = split_costs(D).tile[ks / 2] * (double)(per / unit) +
              (double)ns * (double)rows_total * D * 8.0 / kSplitPartialBytesPerUs;
     return c;
 }
@@ -467,7 +473,7 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
         // At D = 64 / 128 a split of the four-KV-group layout (64 rows per
         // workgroup) is weighed against one of the two-group layout (128 rows,
         // half as many row tiles, twice the partitions): its tiles cost less
-        // (kSplitTileUs), its partials twice as much.  us before -> now at 32 / 8
+        // (SplitCosts), its partials twice as much.  us before -> now at 32 / 8
         // heads, D = 128: 256 x 8192 60.1 -> 54.5, 256 x 16384 107 -> 91.6, 300 x
         // 6000 67.4 -> 51.4, 512 x 16384 (unsplit before) 188 -> 167; D = 64
         // 256 x 8192 40.5 -> 36.4.
@@ -482,8 +488,11 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
                 const long long rt2 = (R + 127) / 128;
                 if (2 * n_groups * rt2 <= cus) {
                     const SplitChoice c = split_prefill(p, n_groups, R, kv_len, D, rows_total, 2, rt2, cus, ws_cap);
-                    const double now = best.ns > 1 ? best.cost : kSplitTileUs[2] * (double)((kv_len + 127) / 128);
-                    if (c.ns > 1 && c.cost + (best.ns > 1 ? kSplitTwoGain : kSplitMergeUs) < now) best = c;
+                    const SplitCosts& us = split_costs(D);
+                    const double now = best.ns > 1 ? best.cost
+                                                   : us.unsplit_tile * (double)((kv_len + 127) / 128) +
+                                                         us.unsplit_kv_mb * 4e-6 * (double)n_groups * kv_len * D;
+                    if (c.ns > 1 && c.cost + (best.ns > 1 ? us.two_gain : us.merge) < now) best = c;
                 }
             }
         }

@@ -84,3 +84,19 @@ def test_partitions_share_a_short_sequences_keys(D):
     parts = p.num_splits * B * H_q * q           # O partials, then the row maxima
     assert torch.isfinite(ws[parts * D:parts * (D + 1)]).all()
     assert torch.equal(kf.attn_fwd(Q, K, V, kv_lens=lens(kv)), kf.attn_fwd(Q, K, V, kv_lens=None))
+
+
+@pytest.mark.parametrize("shape,layout", [
+    # B, q_len, kv_len, H_q, H_kv; us in four groups (split or not), in two
+    ((1, 256, 1024, 32, 8), "8, 4>"),        # 11.8, 13.4
+    ((6, 64, 2048, 32, 8), "8, 4>"),         # 19.3, 22.2
+    ((2, 149, 1741, 32, 1), "8, 4>"),        # 15.9, 17.1
+    ((2, 256, 4096, 32, 8), "8, 4>"),        # 32.5, 34.3
+    ((1, 256, 8192, 32, 8), "8, 2> + kf_attn_split_merge"),   # 36.1, 31.9
+    ((4, 128, 8192, 16, 16), "8, 2> + kf_attn_split_merge"),  # 51.2, 37.1
+])
+def test_d64_takes_the_faster_layout(shape, layout):
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("a GPU is visible: the plan is for its CU count")
+    assert f"kf_attn_prefill_kernel<64, true, {layout}" in kf.kernel_names(*shape, 64, causal=True)
