@@ -131,6 +131,14 @@ size_t kf_attn_workspace_bytes(int B, int q_len, int kv_len, int H_q, int H_kv, 
  * the last bits, within the same tolerance).  No reference counterpart. */
 size_t kf_attn_workspace_bytes_lens(int B, int q_len, int kv_len, int H_q, int H_kv, int D);
 
+/* Bytes of workspace that a caller who has any should give this shape at
+ * least (with or without kv_lens, contiguous or paged): a split decode is
+ * refused with less, a split prefill runs with fewer KV partitions.  0 where
+ * the call is fully split over the compute units without a workspace, though
+ * it may run faster given kf_attn_workspace_bytes() or _lens().  No reference
+ * counterpart. */
+size_t kf_attn_workspace_bytes_least(int B, int q_len, int kv_len, int H_q, int H_kv, int D);
+
 /* Attention forward, asynchronous on `stream`.
  *
  * Replaces launch_once (tests/bench_flash_attn.cu:39-54) and the kernel

@@ -39,7 +39,8 @@ __all__ = [
     "KF_ATTN_CAUSAL",
     "KF_ATTN_OUT_F16", "KF_ATTN_OUT_BF16", "KF_ATTN_LSE",
     "PATH_NAMES", "attn_fwd_ex_ptr", "attn_decode_paged", "attn_decode_paged_ptr",
-    "paged_workspace_bytes", "workspace_bytes_lens", "kernel_names",
+    "paged_workspace_bytes", "workspace_bytes_lens",
+    "workspace_bytes_least", "kernel_names",
 ]
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
@@ -137,8 +138,9 @@ def load_library(path: str = LIB_PATH):
     lib.kf_attn_plan_for_cus.restype = i
     lib.kf_attn_workspace_bytes.argtypes = [i] * 6
     lib.kf_attn_workspace_bytes.restype = sz
-    lib.kf_attn_workspace_bytes_lens.argtypes = [i] * 6
-    lib.kf_attn_workspace_bytes_lens.restype = sz
+    for f in (lib.kf_attn_workspace_bytes_lens, lib.kf_attn_workspace_bytes_least):
+        f.argtypes = [i] * 6
+        f.restype = sz
     lib.kf_attn_kernel_names.argtypes = [i] * 7 + [p, ctypes.c_char_p, sz]
     lib.kf_attn_kernel_names.restype = i
     lib.kf_attn_fwd.argtypes = [p, p, p, p, p, p] + [i] * 6 + [p, sz, p]
@@ -210,6 +212,11 @@ def workspace_bytes(B, q_len, kv_len, H_q, H_kv, D) -> int:
 def workspace_bytes_lens(B, q_len, kv_len, H_q, H_kv, D) -> int:
     """Workspace of a call with kv_lens (kf_attn_workspace_bytes_lens)."""
     return int(load_library().kf_attn_workspace_bytes_lens(B, q_len, kv_len, H_q, H_kv, D))
+
+
+def workspace_bytes_least(B, q_len, kv_len, H_q, H_kv, D) -> int:
+    """Least workspace worth giving a call (kf_attn_workspace_bytes_least)."""
+    return int(load_library().kf_attn_workspace_bytes_least(B, q_len, kv_len, H_q, H_kv, D))
 
 
 def attn_fwd_ptr(Q, K, V, O, Mi, Li, B, q_len, kv_len, H_q, H_kv, D, workspace=0,
@@ -293,20 +300,25 @@ def _output(torch, out, shape, out_dtype, device, stream):
     return out
 
 
-def _workspace(torch, workspace, need, device, stream, required=True):
-    """The split-KV workspace: the caller's if it is a large enough buffer on
-    the device, else a new one (kept alive until ``stream`` passes it).  One
-    on another device is an error where the call cannot do without any
-    (``required``)."""
+def _workspace(torch, workspace, need, least, device, stream):
+    """The split-KV workspace and its bytes: the caller's if it is a buffer on
+    the device of at least ``least()`` bytes (below ``need`` the call runs by
+    a plan that fits), else a new one of ``need`` (kept alive until ``stream``
+    passes it).  One on another device is an error where ``least()`` is not
+    0."""
     if not need:
-        return None
+        return None, 0
     if workspace is not None:
         usable = workspace.device == device and workspace.is_contiguous()
-        if not usable and required:
+        size = workspace.numel() * workspace.element_size() if usable else 0
+        if size >= need:
+            return workspace, need
+        floor = least()
+        if not usable and floor:
             raise ValueError(f"workspace must be a contiguous tensor on {device}")
-        if usable and workspace.numel() * workspace.element_size() >= need:
-            return workspace
-    return _new(torch, need, torch.uint8, device, stream)
+        if usable and size >= floor:
+            return workspace, size
+    return _new(torch, need, torch.uint8, device, stream), need
 
 
 def attn_fwd(Q, K, V, out=None, *, return_stats=False, workspace=None, stream=None,
@@ -318,6 +330,9 @@ def attn_fwd(Q, K, V, out=None, *, return_stats=False, workspace=None, stream=No
     (O, Mi, Li) with ``return_stats``, or (O, LSE) with ``return_lse``.
     Asynchronous on ``stream`` (default: torch's current stream).
     ``causal`` / ``kv_lens`` (int32 GPU tensor [B]) select kf_attn_fwd_ex.
+    ``workspace``: a buffer to use instead of a new one, of workspace_bytes
+    (workspace_bytes_lens with ``kv_lens``) for the fastest run; a smaller one
+    is used too, down to workspace_bytes_least.
     """
     import torch
 
@@ -345,12 +360,10 @@ def attn_fwd(Q, K, V, out=None, *, return_stats=False, workspace=None, stream=No
         Mi = _new(torch, (B, H_q, q_len), torch.float32, Q.device, stream)
     if return_stats:
         Li = _new(torch, (B, H_q, q_len), torch.float32, Q.device, stream)
-    if kv_lens is None:
-        need, required = workspace_bytes(B, q_len, kv_len, H_q, H_kv, D), True
-    else:
-        need = workspace_bytes_lens(B, q_len, kv_len, H_q, H_kv, D)
-        required = workspace is None or workspace_bytes(B, q_len, kv_len, H_q, H_kv, D) > 0
-    workspace = _workspace(torch, workspace, need, Q.device, stream, required)
+    shape = B, q_len, kv_len, H_q, H_kv, D
+    need = workspace_bytes(*shape) if kv_lens is None else workspace_bytes_lens(*shape)
+    workspace, ws_bytes = _workspace(torch, workspace, need, lambda: workspace_bytes_least(*shape),
+                                     Q.device, stream)
     if kv_lens is not None:
         # A contiguous copy would be made on torch's current stream, unordered
         # with a launch on another ``stream``: require the caller's layout.
@@ -365,7 +378,7 @@ def attn_fwd(Q, K, V, out=None, *, return_stats=False, workspace=None, stream=No
                          kv_lens.data_ptr() if kv_lens is not None else 0,
                          (KF_ATTN_CAUSAL if causal else 0) | flags,
                          workspace.data_ptr() if workspace is not None else 0,
-                         need, _raw_stream(torch, stream, Q.device))
+                         ws_bytes, _raw_stream(torch, stream, Q.device))
     if st != KF_OK:
         msg = status_string(st)
         if st == KF_ERR_HIP:
@@ -384,6 +397,7 @@ def attn_decode_paged(Q, K_pages, V_pages, block_table, kv_lens, out=None, *, re
     Q [B, H_q, q_len, D] fp16; K_pages / V_pages [num_pages, H_kv, page_size,
     D] fp16; block_table int32 [B, max_pages_per_seq]; kv_lens int32 [B].
     Returns O [B, H_q, q_len, D] fp32 (and Mi, Li with ``return_stats``).
+    ``workspace`` as in attn_fwd (paged_workspace_bytes).
     """
     import torch
 
@@ -414,7 +428,9 @@ def attn_decode_paged(Q, K_pages, V_pages, block_table, kv_lens, out=None, *, re
     if return_stats:
         Li = _new(torch, (B, H_q, q_len), torch.float32, Q.device, stream)
     need = paged_workspace_bytes(B, q_len, H_q, H_kv, D, page_size, max_pages)
-    workspace = _workspace(torch, workspace, need, Q.device, stream)
+    workspace, ws_bytes = _workspace(
+        torch, workspace, need,
+        lambda: workspace_bytes_least(B, q_len, page_size * max_pages, H_q, H_kv, D), Q.device, stream)
     st = attn_decode_paged_ptr(Q.data_ptr(), K_pages.data_ptr(), V_pages.data_ptr(),
                                block_table.data_ptr(), kv_lens.data_ptr(), out.data_ptr(),
                                Mi.data_ptr() if Mi is not None else 0,
@@ -422,7 +438,7 @@ def attn_decode_paged(Q, K_pages, V_pages, block_table, kv_lens, out=None, *, re
                                B, q_len, H_q, H_kv, D, page_size, max_pages, num_pages,
                                (KF_ATTN_CAUSAL if causal else 0) | flags,
                                workspace.data_ptr() if workspace is not None else 0,
-                               need, _raw_stream(torch, stream, Q.device))
+                               ws_bytes, _raw_stream(torch, stream, Q.device))
     if st != KF_OK:
         msg = status_string(st)
         if st == KF_ERR_HIP:

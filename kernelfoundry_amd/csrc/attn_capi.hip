@@ -305,9 +305,10 @@ void plan_causal(Plan& p, int q_len, int kv_len, int D, int cus) {
 
 // ws_cap: most workspace a split prefill plan may ask for (it then takes
 // fewer KV partitions, or none); split decode plans ignore it, and
-// kf_attn_fwd_noalloc refuses those that exceed its scratch.
+// kf_attn_fwd_noalloc refuses those that exceed its scratch.  two_groups:
+// whether a split prefill may take the two-group layout.
 int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const DeviceShape& dev,
-              Plan* pl, bool paged = false, size_t ws_cap = SIZE_MAX) {
+              Plan* pl, bool paged = false, size_t ws_cap = SIZE_MAX, bool two_groups = true) {
     const int cus = dev.cus;
     if (B <= 0 || q_len <= 0 || kv_len <= 0 || H_q <= 0 || H_kv <= 0 || cus <= 0) return KF_ERR_SIZE;
     if (!supported_head_dim(D)) return KF_ERR_HEAD_DIM;
@@ -477,7 +478,7 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
         // heads, D = 128: 256 x 8192 60.1 -> 54.5, 256 x 16384 107 -> 91.6, 300 x
         // 6000 67.4 -> 51.4, 512 x 16384 (unsplit before) 188 -> 167; D = 64
         // 256 x 8192 40.5 -> 36.4.
-        const bool two = (D == 64 || D == 128) && nw == 8 && ks == 4 && R >= 128;
+        const bool two = two_groups && (D == 64 || D == 128) && nw == 8 && ks == 4 && R >= 128;
         SplitChoice best;
         bool other = false;
         if (p.wide_row_tiles == 0 || D == 256) {
@@ -1048,6 +1049,13 @@ size_t kf_attn_workspace_bytes_lens(int B, int q_len, int kv_len, int H_q, int H
     Plan pl;
     if (make_plan(B, q_len, kv_len, H_q, H_kv, D, current_device_shape(), &pl) != KF_OK) return 0;
     return best_ws_bytes(pl, true);
+}
+
+size_t kf_attn_workspace_bytes_least(int B, int q_len, int kv_len, int H_q, int H_kv, int D) {
+    Plan pl;
+    if (make_plan(B, q_len, kv_len, H_q, H_kv, D, current_device_shape(), &pl, false, SIZE_MAX, false) != KF_OK)
+        return 0;
+    return pl.ws_bytes;
 }
 
 size_t kf_attn_decode_paged_workspace_bytes(int B, int q_len, int H_q, int H_kv, int D,
