@@ -2330,13 +2330,14 @@ __device__ __forceinline__ int seq_keys(const AttnParams& p, int b) {
 }
 __device__ __forceinline__ int key_stages(int keys) { return (keys + kDecodeStage - 1) / kDecodeStage; }
 
-// Inclusive prefix sum over the lanes.
-__device__ __forceinline__ int wave_scan(int v, int lane) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int u = __shfl_up(v, d);
-        if (lane >= d) v += u;
-    }
+// Inclusive prefix sum over the lanes, by row shifts and row broadcasts.
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 to rows 1, 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2, 3
     return v;
 }
 
@@ -2361,43 +2362,101 @@ struct RaggedSeg {
     int T, kvb;   // stages and keys of the head
 };
 
-// The stages of all sequences.  The first 64 sequences' keys and prefix sums
-// stay in registers, a lane each; larger batches re-read the others.
+// The stages of all sequences, for lookups at increasing positions.  Up to 256
+// sequences' keys and prefix sums are in registers, 64 to a register; of a
+// larger batch those of 64 that the last lookup fell among.  Where to look for
+// others is known from the stages of 64 blocks of sequences, which the
+// workgroup's waves count together.  (Counting through the batch from its
+// start, in every wave and for every lookup, 4096 sequences of 16 to 256 keys
+// at one KV head, D = 64, took 181 us, and 51 so.)
 struct RaggedMap {
-    int keys, inc;   // this lane's sequence: keys, stages per head up to and with it
-    int total;       // stages of all heads (the host keeps it within int)
+    // 64 sequences, a lane each: keys, stages per head up to and with it.
+    struct Regs {
+        int keys, inc;
+    };
+    int total;          // stages of all heads (the host keeps it within int)
+    int block;          // sequences per block, a multiple of 64; 0: all are in registers
+    int block_inc;      // this lane's block: stages per head up to and with it
+    int base, before;   // first sequence in registers, stages per head before it
+    Regs r0, r1, r2, r3;  // sequences from base on (r1 .. r3: base 0, small batches)
 
-    __device__ __forceinline__ void init(const AttnParams& p, int lane) {
-        keys = seq_keys(p, lane);
-        inc = wave_scan(key_stages(keys), lane);
-        int sum = __builtin_amdgcn_readlane(inc, 63);
-        for (int b0 = 64; b0 < p.batch; b0 += 64)
-            sum += __builtin_amdgcn_readlane(wave_scan(key_stages(seq_keys(p, b0 + lane)), lane), 63);
+    // Sequences [b, b + 64) of the first `stop`, `sum` stages per head before
+    // them; adds theirs.
+    static __device__ __forceinline__ Regs load(const AttnParams& p, int lane, int b, int stop, int& sum) {
+        Regs r{0, sum};
+        if (b < stop) {
+            r.keys = b + lane < stop ? seq_keys(p, b + lane) : 0;
+            r.inc += wave_scan(key_stages(r.keys));
+            sum = __builtin_amdgcn_readlane(r.inc, 63);
+        }
+        return r;
+    }
+
+    // blocks: LDS for 64 counts.
+    __device__ __forceinline__ void init(const AttnParams& p, int lane, int wave, int waves, int* blocks) {
+        base = before = block = block_inc = 0;
+        int sum = 0;
+        r0 = r1 = r2 = r3 = Regs{0, 0};
+        if (p.batch <= 256) {
+            r0 = load(p, lane, 0, p.batch, sum);
+            r1 = load(p, lane, 64, p.batch, sum);
+            r2 = load(p, lane, 128, p.batch, sum);
+            r3 = load(p, lane, 192, p.batch, sum);
+        } else {
+            block = (p.batch + 64 * 64 - 1) / (64 * 64) * 64;
+            for (int k = wave; k < 64; k += waves) {
+                int n = 0;
+                for (int b = k * block + lane; b < min((k + 1) * block, p.batch); b += 64)
+                    n += key_stages(seq_keys(p, b));
+                n = wave_scan(n);
+                if (lane == 63) blocks[k] = n;
+            }
+            __syncthreads();
+            block_inc = wave_scan(blocks[lane]);
+            sum = __builtin_amdgcn_readlane(block_inc, 63);
+        }
         total = sum * p.heads_kv;
     }
     // The segment that starts at global stage pos (pos < end <= total).
-    __device__ __forceinline__ RaggedSeg find(const AttnParams& p, int lane, int pos, int end) const {
-        RaggedSeg s{0, 0, 0, 0, 1, 0};
-        int k64 = keys, i64 = inc, carry = 0;
-        for (int b0 = 0;;) {
-            // Sequences whose stages all lie before pos come first.
-            const int k = __popcll(__ballot((carry + i64) * p.heads_kv <= pos));
-            if (k < 64) {
-                s.b = b0 + k;
-                s.kvb = __builtin_amdgcn_readlane(k64, k);
-                s.T = key_stages(s.kvb);
-                const int off = pos - (carry + __builtin_amdgcn_readlane(i64, k) - s.T) * p.heads_kv;
-                s.h = __builtin_amdgcn_readfirstlane(off / s.T);
-                s.t0 = off - s.h * s.T;
-                s.n = min(s.T - s.t0, end - pos);
-                return s;
+    __device__ __forceinline__ RaggedSeg find(const AttnParams& p, int lane, int pos, int end) {
+        // Sequences in registers whose stages all lie before pos.
+        const auto passed = [&](const Regs& r) { return __popcll(__ballot((before + r.inc) * p.heads_kv <= pos)); };
+        int k = passed(r0);
+        Regs r = r0;
+        if (k == 64 && block == 0) {
+            if (const int n = passed(r1); n < 64) {
+                k += n;
+                r = r1;
+            } else if (const int n = passed(r2); n < 64) {
+                k += 64 + n;
+                r = r2;
+            } else {
+                k += 128 + passed(r3);
+                r = r3;
             }
-            carry += __builtin_amdgcn_readlane(i64, 63);
-            b0 += 64;
-            if (b0 >= p.batch) return s;  // not reached
-            k64 = seq_keys(p, b0 + lane);
-            i64 = wave_scan(key_stages(k64), lane);
+        } else if (k == 64) {
+            const int at = __popcll(__ballot(block_inc * p.heads_kv <= pos));
+            const int stop = min((at + 1) * block, p.batch);
+            before = at > 0 ? __builtin_amdgcn_readlane(block_inc, at - 1) : 0;
+            for (base = at * block;; base += 64) {
+                int sum = 0;
+                r0 = load(p, lane, base, stop, sum);
+                k = passed(r0);
+                if (k < 64 || base + 64 >= stop) break;
+                before += sum;
+            }
+            r = r0;
         }
+        RaggedSeg s{0, 0, 0, 0, 1, 0};
+        s.b = base + k;
+        if (s.b >= p.batch) return s;  // not reached
+        s.kvb = __builtin_amdgcn_readlane(r.keys, k & 63);
+        s.T = key_stages(s.kvb);
+        const int off = pos - (before + __builtin_amdgcn_readlane(r.inc, k & 63) - s.T) * p.heads_kv;
+        s.h = __builtin_amdgcn_readfirstlane(off / s.T);
+        s.t0 = off - s.h * s.T;
+        s.n = min(s.T - s.t0, end - pos);
+        return s;
     }
 };
 
@@ -2428,8 +2487,9 @@ void kf_attn_decode_ragged_kernel(AttnParams p) {
     const int row = lane & 31;
     const int R = p.rows_per_group;
     const int wg = blockIdx.x;
+    __shared__ int blocks[64];
     RaggedMap map;
-    map.init(p, lane);
+    map.init(p, lane, wave, NW, blocks);
     // Merged: the stages go to the workgroups (as many as leave each of their
     // waves one) and from them to their waves.
     // Spread: straight to all waves, the first of every workgroup first.

@@ -3,8 +3,8 @@ waves share the stages that the sequences really hold.
 
 Shapes where the division can go wrong: empty sequences and single keys, one
 long sequence among short ones (a head over many workers), hundreds of heads
-inside one worker's share, more than 64 sequences (the batch map's second
-round), counts past the capacity, 1 to 16 rows per KV head (both ways of
+inside one worker's share, more than 64 and 192 sequences (the batch map's
+registers), more than 256 and 4096 (its blocks, of 64 and 128), counts past the capacity, 1 to 16 rows per KV head (both ways of
 merging), every head dimension, page sizes from 16 rows, invalid page ids.
 Bar as in the other parity tests (fp64 oracle), and the same call by the
 capacity's splits (a workspace of only kf_attn_workspace_bytes) within 2e-4:
@@ -49,6 +49,12 @@ CASES = [
     (96, 4, 2, 3, 4096, 16, 16, "one_long", True),
     (16, 16, 4, 1, 4096, 256, 16, "mixed", False),
     (16, 16, 4, 3, 4096, 256, 0, "one_long", True),    # 12 rows
+    (256, 8, 2, 1, 512, 128, 16, "mixed", False),      # the registers' last sequence
+    (257, 8, 2, 1, 512, 128, 0, "mixed", False),       # one block more than them
+    (700, 4, 2, 3, 300, 64, 0, "one_long", True),
+    (1000, 16, 4, 1, 200, 256, 0, "short", False),
+    (4500, 4, 2, 1, 64, 16, 16, "short", False),       # blocks of 128 sequences
+    (4500, 4, 2, 1, 64, 16, 0, "one_long", False),
 ]
 
 
