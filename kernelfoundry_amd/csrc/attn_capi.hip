@@ -185,8 +185,8 @@ struct Plan {
     int wide_kv_groups; // KV groups of the wide kernel (2: D = 256, 128 rows per workgroup)
     bool wide_causal;   // D = 64 / 128: causal calls take the wide kernel too
     // Unsplit causal calls that take neither that nor the plan above (0 waves:
-    // they take it): waves, KV groups, the groups the 8-wave kernel makes of
-    // one (kf_attn_prefill_kernel), and the 128-row KV-group kernel at D = 256.
+    // they take it): waves, KV groups, 2 for the 8-wave kernel's two-group form
+    // (kf_attn_prefill_kernel), and the 128-row KV-group kernel at D = 256.
     int causal_waves, causal_kv_groups, causal_groups;
     bool causal_wide2;
     int short_stages;   // decode: 32-key stages per split of the short-split kernel, 0 = streaming kernel
@@ -573,16 +573,23 @@ hipError_t launch_prefill_kernel(const Plan& plan, const kf::AttnParams& params,
             pl.wide_kv_groups = 2;
         } else if (pl.causal_groups == 2) {
             tiles(128);
-            prm.causal_groups = 2;
         } else if (pl.causal_waves > 0) {
             pl.waves = pl.causal_waves;
             pl.kv_groups = pl.causal_kv_groups;
             pl.threads = 64 * pl.waves;
             tiles(32 * pl.waves / pl.kv_groups);
         }
-        // (The divisions of causal_place and causal_tile take up to 0.5 us of
-        // a small call: 4 x 150 queries, MQA at D = 128, 10.46 us without, 10.92 with.)
-        prm.causal_one_round = std::max(pl.grid, pl.wide_row_tiles > 0 ? pl.wide_grid : 0) <= pl.cus;
+        // The order of the row tiles.  The divisions of causal_place and
+        // causal_tile take up to 0.7 us of a call, so a grid of one round, heads of
+        // a tile or so and rows that see nearly equal counts go from each KV
+        // head's last tile down, and so does one query head per KV head, for which
+        // that is causal_tile's order (4 x 576 queries at 16 / 16 heads, D = 64
+        // 17.9 us by causal_tile, 17.3 so; 2 x 100 at 32 / 8, D = 128 7.50, 7.33).
+        // 8 x 500 at 32 / 8 heads, D = 128 48.5 so, 44.2 by causal_tile.
+        if (std::max(pl.grid, pl.wide_row_tiles > 0 ? pl.wide_grid : 0) > pl.cus) {
+            const bool by_tile = pl.R > prm.q_len && prm.q_len >= 256 && 4LL * prm.q_len > prm.kv_len;
+            prm.causal_order = by_tile ? 2 : prm.causal_sets != prm.xcds ? 1 : 0;
+        }
     }
     if constexpr (D >= 256) {
         if (pl.wide_row_tiles > 0) {
@@ -617,6 +624,11 @@ hipError_t launch_prefill_kernel(const Plan& plan, const kf::AttnParams& params,
             }
         }
         if constexpr (D == 64 || D == 128) {
+            if (prm.causal && pl.causal_groups == 2) {
+                kf::kf_attn_prefill_kernel<D, true, 8, 1>
+                    <<<dim3(pl.grid), dim3(pl.threads), 0, stream>>>(kf::AttnTwoGroups{prm});
+                return hipGetLastError();
+            }
             // Causal calls take the wide layout's causal kernel when its grid
             // balances (wide_causal), else the 256-row kernel.
             if (pl.wide_row_tiles > 0 && (!prm.causal || pl.wide_causal)) {

@@ -129,12 +129,15 @@ struct AttnParams {
     // the dispatcher deals workgroup ids round-robin over them.
     int xcds;
     int causal_sets, causal_per;  // causal_place: sets of KV heads and XCDs, heads per set
-    int causal_one_round;  // a workgroup per CU at most: no order, the plain placement
-    int causal_groups;  // KV groups of the causal 8-wave kernel (1 or 2)
+    int causal_order;  // row tiles: 0 from a KV head's last, 1 the same on causal_place, 2 by causal_tile
     // Ragged decode (kf_attn_decode_ragged_kernel).
     int batch;
     u32x4* ragged_heads;     // [B * H_kv] where a head's partials are
 };
+
+// Selects the two-group form of the causal 8-wave kernel (by the type of the
+// kernel's argument: a kernel of its own under the same name).
+struct AttnTwoGroups : AttnParams {};
 
 enum : int { kOutF32 = 0, kOutF16 = 1, kOutBF16 = 2 };
 // Internal store target of the split prefill: fp32 partial O at p.Opart.
@@ -272,7 +275,7 @@ __device__ __forceinline__ int causal_tile(int k, int row_tiles, int heads, int 
 // 4-wave workgroups 53.1 us so, 36.3 alternating.)
 constexpr int kCausalMix = 4;
 __device__ __forceinline__ void causal_place(int hw, int tiles, int sets, int per, int& grp, int& k) {
-    asm volatile("" ::: "memory");  // a branch of its own, not computed by every call
+    asm volatile("");  // a branch of its own, not computed by every call
     const int s = hw & (sets - 1), m = hw >> __builtin_ctz(sets);
     if (per <= kCausalMix) {
         k = m / per;
@@ -1022,10 +1025,13 @@ __device__ __forceinline__ void prefill_body(AttnParams p, char* buf0, char* buf
     const float c = p.scale_log2;
     if (kMask && p.causal) {
         // (One XCD per set: xcd_remap's ranges are the same.)
-        if (__builtin_expect(!p.causal_one_round, 0)) {  // (out of the small calls' code)
+        if (__builtin_expect(p.causal_order != 0, 0)) {  // (out of the small calls' code)
             if (nsp == 1 && p.causal_sets != p.xcds)
                 causal_place(blockIdx.x, p.row_tiles, p.causal_sets, p.causal_per, grp, rt);
-            rt = causal_tile(rt, p.row_tiles, R / p.q_len, p.q_len, kPrefillRows);
+            rt = p.causal_order == 2 ? causal_tile(rt, p.row_tiles, R / p.q_len, p.q_len, kPrefillRows)
+                                     : p.row_tiles - 1 - rt;
+        } else {
+            rt = p.row_tiles - 1 - rt;
         }
     }
 
@@ -1447,32 +1453,36 @@ __device__ __forceinline__ void prefill_body(AttnParams p, char* buf0, char* buf
     }
 }
 
-// kTwo (the causal 8-wave kernel at D = 64 / 128): with p.causal_groups == 2
-// the workgroup takes 128 rows in two KV groups instead of 256 rows in one.  A
-// causal grid of one round of 256-row tiles lasts as long as its longest tile,
-// while the average row sees half its keys; twice as many tiles whose keys two
-// groups share halve the longest chain and fill the CUs longest first.  S =
-// 2048 at 32 / 8 heads: 67.4 -> 58 us (D = 128), 46.9 -> 39.5 (D = 64).
 template <int D, bool kMask, int NW = kPrefillMaxWaves<D>, int KS = 1>
 __global__ __launch_bounds__((PrefillCfg<D, NW, KS>::kThreads), (PrefillCfg<D, NW, KS>::kWavesPerEU))
 void kf_attn_prefill_kernel(AttnParams p) {
-    constexpr bool kTwo = kMask && NW == 8 && KS == 1 && (D == 64 || D == 128);
     using L = PrefillLds<D, NW, KS>;
-    using L2 = PrefillLds<D, NW, kTwo ? 2 : KS>;
-    constexpr auto most = [](int a, int b) { return a > b ? a : b; };
-    __shared__ __attribute__((aligned(1024))) char buf0[most(L::kBuf, L2::kBuf)];
-    __shared__ __attribute__((aligned(1024))) char buf1[most(L::kBuf, L2::kBuf)];
-    __shared__ __attribute__((aligned(1024))) char buf2[most(L::kBuf2, L2::kBuf2)];
+    __shared__ __attribute__((aligned(1024))) char buf0[L::kBuf];
+    __shared__ __attribute__((aligned(1024))) char buf1[L::kBuf];
+    __shared__ __attribute__((aligned(1024))) char buf2[L::kBuf2];
     __shared__ __attribute__((aligned(16))) char zero_pad[16];  // D=16: V^T rows 16..31
-    __shared__ __attribute__((aligned(1024))) char q_lds[most(L::kQ, L2::kQ)];
-    __shared__ float merge_ml[most(L::kMl, L2::kMl)];
-    if constexpr (kTwo) {
-        if (p.causal_groups == 2) {
-            prefill_body<D, kMask, NW, 2, (D <= 128)>(p, buf0, buf1, buf2, zero_pad, q_lds, merge_ml);
-            return;
-        }
-    }
+    __shared__ __attribute__((aligned(1024))) char q_lds[L::kQ];
+    __shared__ float merge_ml[L::kMl];
     prefill_body<D, kMask, NW, KS, (D <= 128)>(p, buf0, buf1, buf2, zero_pad, q_lds, merge_ml);
+}
+
+// The causal 8-wave kernel at D = 64 / 128 with 128 rows in two KV groups
+// instead of 256 rows in one.  A causal grid of one round of 256-row tiles
+// lasts as long as its longest tile, while the average row sees half its keys;
+// twice as many tiles whose keys two groups share halve the longest chain and
+// fill the CUs longest first.  S = 2048 at 32 / 8 heads: 67.4 -> 58 us (D =
+// 128), 46.9 -> 39.5 (D = 64).
+template <int D, bool kMask, int NW, int KS>
+__global__ __launch_bounds__((PrefillCfg<D, NW, 2>::kThreads), (PrefillCfg<D, NW, 2>::kWavesPerEU))
+void kf_attn_prefill_kernel(AttnTwoGroups p) {
+    static_assert(kMask && NW == 8 && KS == 1 && (D == 64 || D == 128), "the causal 8-wave kernel");
+    using L = PrefillLds<D, NW, 2>;
+    __shared__ __attribute__((aligned(1024))) char buf0[L::kBuf];
+    __shared__ __attribute__((aligned(1024))) char buf1[L::kBuf];
+    __shared__ __attribute__((aligned(1024))) char buf2[L::kBuf2];
+    __shared__ __attribute__((aligned(1024))) char q_lds[L::kQ];
+    __shared__ float merge_ml[L::kMl];
+    prefill_body<D, kMask, NW, 2, false>(p, buf0, buf1, buf2, nullptr, q_lds, merge_ml);
 }
 
 // The split prefill at D = 256: the 4-wave kernel with KV partitions.
@@ -1596,10 +1606,13 @@ void kf_attn_prefill_wide_kernel(AttnParams p) {
     const int kv_len = p.kv_len;
     const float c = p.scale_log2;
     if (causal) {
-        if (__builtin_expect(!p.causal_one_round, 0)) {  // (out of the small calls' code)
+        if (__builtin_expect(p.causal_order != 0, 0)) {  // (out of the small calls' code)
             if (p.causal_sets != p.xcds)
                 causal_place(blockIdx.x, p.row_tiles, p.causal_sets, p.causal_per, grp, rt);
-            rt = causal_tile(rt, p.row_tiles, R / p.q_len, p.q_len, kRows);
+            rt = p.causal_order == 2 ? causal_tile(rt, p.row_tiles, R / p.q_len, p.q_len, kRows)
+                                     : p.row_tiles - 1 - rt;
+        } else {
+            rt = p.row_tiles - 1 - rt;
         }
     }
     // Keys this workgroup needs (blk_lim) and, per wave, the smallest row
