@@ -581,14 +581,23 @@ hipError_t launch_prefill_kernel(const Plan& plan, const kf::AttnParams& params,
         }
         // The order of the row tiles.  The divisions of causal_place and
         // causal_tile take up to 0.7 us of a call, so a grid of one round, heads of
-        // a tile or so and rows that see nearly equal counts go from each KV
+        // a tile or so in up to two and rows that see nearly equal counts go from each KV
         // head's last tile down, and so does one query head per KV head, for which
         // that is causal_tile's order (4 x 576 queries at 16 / 16 heads, D = 64
         // 17.9 us by causal_tile, 17.3 so; 2 x 100 at 32 / 8, D = 128 7.50, 7.33).
         // 8 x 500 at 32 / 8 heads, D = 128 48.5 so, 44.2 by causal_tile.
-        if (std::max(pl.grid, pl.wide_row_tiles > 0 ? pl.wide_grid : 0) > pl.cus) {
-            const bool by_tile = pl.R > prm.q_len && prm.q_len >= 256 && 4LL * prm.q_len > prm.kv_len;
-            prm.causal_order = by_tile ? 2 : prm.causal_sets != prm.xcds ? 1 : 0;
+        const int grid = std::max(pl.grid, pl.wide_row_tiles > 0 ? pl.wide_grid : 0);
+        if (grid > pl.cus) {
+            const bool by_tile = pl.R > prm.q_len && 4LL * prm.q_len > prm.kv_len &&
+                                 (prm.q_len >= 256 || grid > 2LL * pl.cus);
+            // One query head per KV head: on causal_place where it deals a set's
+            // heads side by side (1 x 4096 at 12 / 12 heads, D = 128 83.7 -> 74 us;
+            // one after the other, XCDs that share a head take its longer and its
+            // shorter tiles, 9 x 1024 at 4 / 4 heads 37 -> 43, 9 x 2000 at 2 / 2,
+            // D = 256 98 -> 149).
+            const bool side_by_side = pl.R == prm.q_len && prm.causal_sets != prm.xcds &&
+                                      prm.causal_per <= kf::kCausalMix;
+            prm.causal_order = by_tile ? 2 : side_by_side ? 1 : 0;
         }
     }
     if constexpr (D >= 256) {
