@@ -297,6 +297,26 @@ void plan_causal(Plan& p, int q_len, int kv_len, int D, int cus) {
     const bool straddle = q_len % 256 != 0;
     const int groups = D == 64 && kv_len >= kMinGroupKeys ? 2 : 1;
     if (p.grid <= cus && groups == 1) return;
+    // D = 64: a key takes 4 % longer in the 64-row tiles (22 rounds of 2040 keys
+    // 724 against 760 us), which their waste has to be worth: 256-row tiles that
+    // pad 2 % more rows; tiles that straddle several query heads, which share K
+    // and V, up to three rounds (eight from eight heads on); or one head whose
+    // 64-row tiles, three to a CU, fill their rounds where 256-row tiles do not.
+    // 16 / 16 heads: 8 x 400 queries, one full round, 12.7 us against 15.9; 11 x
+    // 713 36.5 against 43.4; but 8 x 700 32.0 against 30.2, 9 x 1024 69.4 against
+    // 55.3.  32 / 8 heads 14 x 768 81 against 85, 3 x 900 41 against 28.6.  MQA
+    // 7 x 2026 224 against 206, 16 x 256 21.2 against 23.8.
+    if (groups == 2) {
+        const int heads = p.R / q_len;
+        const long long padded256 = (p.R + 255LL) / 256 * 256, padded64 = (p.R + 63LL) / 64 * 64;
+        const auto fill = [](long long grid, long long slots) {
+            return (double)grid / (double)((grid + slots - 1) / slots * slots);
+        };
+        const bool pays = 50 * padded256 >= 51 * padded64 ||
+                          (straddle && heads > 1 && p.grid <= (heads >= 8 ? 8LL : 3LL) * cus) ||
+                          (heads == 1 && fill(p.grid, cus) <= 0.9 && fill(grid_of(64), 3LL * cus) >= 0.98);
+        if (!pays || (p.grid <= cus && 2 * avg_keys < kCausalShortKeys)) return;
+    }
     if (avg_keys < (straddle ? kWideCausalMinKeys : kCausalShortKeys) && grid_of(64) <= INT_MAX) {
         p.causal_waves = 4;
         p.causal_kv_groups = groups;

@@ -29,6 +29,16 @@ CASES = [
     (4, 32, 8, 1024, 700, 128, PREFILL.format(128, 8, 1)),    # fewer keys than queries: as before
     (2, 32, 1, 300, 300, 128, PREFILL.format(128, 4, 2)),     # 2 KV heads, 64-row tiles, ragged
     (3, 2, 1, 5000, 5000, 64, PREFILL.format(64, 8, 4)),      # long rows, 3 heads
+    # One query head per KV head, 12 of them (4 sets of 3, side by side) and 36
+    # (4 sets of 9, the plain placement).
+    (1, 12, 12, 5900, 5900, 128, PREFILL.format(128, 8, 1)),
+    (3, 12, 12, 2048, 2048, 128, PREFILL.format(128, 8, 1)),
+    # D = 64: full rounds of 256-row tiles, tiles that do not straddle, tiles that pad.
+    (8, 16, 16, 400, 400, 64, PREFILL.format(64, 8, 1)),
+    (16, 32, 1, 256, 256, 64, PREFILL.format(64, 8, 1)),
+    (8, 16, 16, 700, 700, 64, PREFILL.format(64, 4, 2)),
+    (9, 16, 16, 1024, 1024, 64, PREFILL.format(64, 4, 2)),
+    (11, 16, 16, 713, 713, 64, PREFILL.format(64, 8, 1)),
 ]
 
 
@@ -56,7 +66,7 @@ def test_parity(case, lens):
     Q, K, V = (torch.randn((B, h, n, D), generator=g, dtype=torch.float16, device="cuda")
                for h, n in ((H_q, q), (H_kv, kv), (H_kv, kv)))
     # Key counts below kv_len, the last below q_len (rows without keys).
-    counts = [kv - 37 * (b + 1) if b < B - 1 else min(kv, q) // 3 for b in range(B)] if lens else [kv] * B
+    counts = [max(kv - 37 * (b + 1), 5) if b < B - 1 else min(kv, q) // 3 for b in range(B)] if lens else [kv] * B
     L = torch.tensor(counts, dtype=torch.int32, device="cuda") if lens else None
     O, Mi, Li = kf.attn_fwd(Q, K, V, causal=True, kv_lens=L, return_stats=True)
     ratio = H_q // H_kv
