@@ -126,6 +126,9 @@ constexpr int kRaggedMaxRows = 16;
 // 8 x 4096 at 16 / 4 heads 37.7 -> 31.7.  Of several rounds the least gain was
 // 24 x 8192 keys, 129.7 -> 130.3.
 constexpr int kRaggedEvenRows = 8;
+// Waves of its merge, beyond which heads of many partials share (25 x 2 queries,
+// 64 / 8 heads: 22.1 us, with 4096 23.8, with 2048 26.8; large batches alike).
+constexpr int kRaggedMergeMaxWaves = 8192;
 constexpr int kCausalShortKeys = 768;
 constexpr int kCausalWide2Keys = 1024;
 constexpr size_t kWsAlign = 256;
@@ -749,7 +752,12 @@ hipError_t launch_merge(const Plan& pl, const kf::AttnParams& prm, hipStream_t s
 
 // The ragged decode and its merge (one wave per query row and column block).
 template <int D>
-hipError_t launch_ragged(const Plan& pl, const kf::AttnParams& prm, hipStream_t stream) {
+hipError_t launch_ragged(const Plan& pl, const kf::AttnParams& params, hipStream_t stream) {
+    kf::AttnParams prm = params;
+    // A wave per item of a head of many partials, up to kRaggedMergeMaxWaves in
+    // all; then as many as cover the rows of one of few.
+    const int items = pl.R * kf::RaggedMerge<D>::kNCB, few = (pl.R * (D / 4) + 63) / 64;
+    prm.merge_waves = std::max(few, std::min(items, kRaggedMergeMaxWaves / pl.n_groups));
     const dim3 grid(pl.ragged_wgs), block(kf::RaggedCfg<D>::kThreads);
     if (prm.block_table)
         kf::kf_attn_decode_ragged_kernel<D, true><<<grid, block, 0, stream>>>(prm);
@@ -757,9 +765,9 @@ hipError_t launch_ragged(const Plan& pl, const kf::AttnParams& prm, hipStream_t 
         kf::kf_attn_decode_ragged_kernel<D, false><<<grid, block, 0, stream>>>(prm);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    constexpr int kPerRow = (D / 4 + kf::kRaggedMergeCols - 1) / kf::kRaggedMergeCols, kWaves = kf::kRaggedMergeWaves;
-    const int blocks = (int)(((long long)pl.rows_total * kPerRow + kWaves - 1) / kWaves);
-    kf::kf_attn_ragged_merge_kernel<D><<<dim3(blocks), dim3(64 * kWaves), 0, stream>>>(prm);
+    constexpr int kWaves = kf::kRaggedMergeWaves;
+    const long long blocks = ((long long)pl.n_groups * prm.merge_waves + kWaves - 1) / kWaves;
+    kf::kf_attn_ragged_merge_kernel<D><<<dim3((unsigned)blocks), dim3(64 * kWaves), 0, stream>>>(prm);
     return hipGetLastError();
 }
 

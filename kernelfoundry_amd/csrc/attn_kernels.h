@@ -132,6 +132,7 @@ struct AttnParams {
     int causal_order;  // row tiles: 0 from a KV head's last, 1 the same on causal_place, 2 by causal_tile
     // Ragged decode (kf_attn_decode_ragged_kernel).
     int batch;
+    int merge_waves;         // waves per KV head of its merge
     u32x4* ragged_heads;     // [B * H_kv] where a head's partials are
 };
 
@@ -2883,77 +2884,122 @@ void kf_attn_decode_ragged_kernel(AttnParams p) {
     }
 }
 
-// Merge of the ragged decode's partials: one wave per (query row, block of CW
-// float4 columns), 64 / CW split lanes.  A head's partials are the one of the
-// worker (spread) or the merged one of the workgroup where it starts, one of
-// each further worker or workgroup (in its first worker's slot), and at most
-// one that a workgroup's worker wrote by itself.
-// A head whose rows are final is left; a sequence without keys gets O = 0,
-// Mi = -inf, Li = 0 here.
+// Merge of the ragged decode's partials, p.merge_waves waves per KV head.  A
+// head's partials are the one of the worker (spread) or the merged one of the
+// workgroup where it starts, one of each further worker or workgroup (in its
+// first worker's slot), and at most one that a workgroup's worker wrote by
+// itself.  A head whose rows are final is left; a sequence without keys gets
+// O = 0, Mi = -inf, Li = 0 here.
+//
+// Latency: the table's entry, then the partials, all of an item's loads in
+// flight.  Up to kRaggedFew partials, as the many heads of a large batch have:
+// a lane per float4 column of the rows.  More of them: a wave per (row, block
+// of CW columns), 64 / CW split lanes.  (That wave for every row, whatever the
+// count, took 47 us for 12800 rows of two partials at D = 256, 200 x 4 queries
+// against 704 keys at 16 / 4 heads; the call went from 157 to 124 us.)
 constexpr int kRaggedMergeCols = 8;
 constexpr int kRaggedMergeWaves = 4;
+constexpr int kRaggedFew = 4;
+template <int D> struct RaggedMerge {
+    static constexpr int CW = D / 4 < kRaggedMergeCols ? D / 4 : kRaggedMergeCols;
+    static constexpr int kNCB = (D / 4) / CW;         // column blocks per row
+};
 template <int D>
 __global__ __launch_bounds__(64 * kRaggedMergeWaves)
 void kf_attn_ragged_merge_kernel(AttnParams p) {
-    constexpr int CW = D / 4 < kRaggedMergeCols ? D / 4 : kRaggedMergeCols;
-    constexpr int kNCB = (D / 4) / CW;                // column blocks per row
+    constexpr int CW = RaggedMerge<D>::CW, kNCB = RaggedMerge<D>::kNCB;
     constexpr int kSL = 64 / CW;                      // split lanes per column
     constexpr int kUnroll = 4;
     const int lane = threadIdx.x & 63;
     const int wid = blockIdx.x * kRaggedMergeWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int ri = wid / kNCB, cb = wid % kNCB;
-    if (ri >= p.rows_total) return;
+    const int waves = p.merge_waves;
+    const int grp = wid / waves, part = wid - grp * waves;
+    if (grp >= p.batch * p.heads_kv) return;
     const int R = p.rows_per_group;
-    const int grp = ri / R, r = ri - grp * R;
     const u32x4 head = p.ragged_heads[grp];           // not written for a sequence without keys
     const bool empty = seq_keys(p, grp / p.heads_kv) == 0;
     const int groups = empty ? 0 : (int)head.y;
     const int ns = empty ? 0 : groups + ((int)head.z >= 0 ? 1 : 0);
     if (ns == 1) return;
     const int stride = (int)head.w, first = (int)head.x / max(stride, 1);
-    const int c = cb * CW + lane % CW, sl = lane / CW;
-
-    float m = -INFINITY, l = 0.f;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = sl; k0 < ns; k0 += kSL * kUnroll) {
-        f32x4 ov[kUnroll];
-        float mv[kUnroll], lv[kUnroll];
+    auto partial = [&](int k, int r) {                // of row r
+        const int slot = k == 0 ? (int)head.x : k < groups ? (first + k) * stride : (int)head.z;
+        return (size_t)slot * R + r;
+    };
+    if (ns <= kRaggedFew) {
+        for (int i = part * 64 + lane; i < R * (D / 4); i += waves * 64) {
+            const int r = i / (D / 4), c = i % (D / 4);
+            f32x4 ov[kRaggedFew], acc = {0.f, 0.f, 0.f, 0.f};
+            float mv[kRaggedFew], lv[kRaggedFew], m = -INFINITY, l = 0.f;
+            if (ns > 0) {
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            const int k = min(k0 + u * kSL, ns - 1);
-            const int slot = k == 0 ? (int)head.x : k < groups ? (first + k) * stride : (int)head.z;
-            const size_t pi = (size_t)slot * R + r;
-            ov[u] = *reinterpret_cast<const f32x4*>(p.Opart + pi * D + 4 * c);
-            mv[u] = p.Mpart[pi];
-            lv[u] = p.Lpart[pi];
+                for (int k = 0; k < kRaggedFew; ++k) {
+                    const size_t pi = partial(min(k, ns - 1), r);
+                    ov[k] = *reinterpret_cast<const f32x4*>(p.Opart + pi * D + 4 * c);
+                    mv[k] = p.Mpart[pi];
+                    lv[k] = p.Lpart[pi];
+                }
+#pragma unroll
+                for (int k = 0; k < kRaggedFew; ++k) m = fmaxf(m, mv[k]);
+#pragma unroll
+                for (int k = 0; k < kRaggedFew; ++k) {
+                    const bool in = k < ns;
+                    const float w = in && m != -INFINITY ? exp2_hw((mv[k] - m) * kLog2e) : 0.f;  // 0 keeps a NaN
+                    l += in ? w * lv[k] : 0.f;
+                    acc += in ? w * ov[k] : f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+            }
+            const size_t ri = (size_t)grp * R + r;
+            store_out4(p, ri * D + 4 * c, acc * (l > 0.f ? 1.0f / l : 0.f));
+            if (c == 0) store_stats(p, ri, m, l);
         }
-        float mx = m;
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) mx = fmaxf(mx, mv[u]);
-        const bool none = mx == -INFINITY;            // weight 0 below keeps a NaN
-        const float keep = none ? 1.f : exp2_hw((m - mx) * kLog2e);
-        acc *= keep;
-        l *= keep;
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            const bool in = k0 + u * kSL < ns;
-            const float w = in && !none ? exp2_hw((mv[u] - mx) * kLog2e) : 0.f;
-            l += in ? w * lv[u] : 0.f;
-            acc += in ? w * ov[u] : f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        m = mx;
+        return;
     }
-    const float mm = reduce_mod<CW, true>(m);
-    const float w = mm == -INFINITY ? 0.f : exp2_hw((m - mm) * kLog2e);
-    l = reduce_mod<CW, false>(l * w);
-    acc *= w;
-    acc.x = reduce_mod<CW, false>(acc.x);
-    acc.y = reduce_mod<CW, false>(acc.y);
-    acc.z = reduce_mod<CW, false>(acc.z);
-    acc.w = reduce_mod<CW, false>(acc.w);
-    if (sl == 0) {
-        store_out4(p, (size_t)ri * D + 4 * c, acc * (l > 0.f ? 1.0f / l : 0.f));
-        if (c == 0) store_stats(p, ri, mm, l);
+    const int sl = lane / CW;
+    for (int item = part; item < R * kNCB; item += waves) {
+        const int r = item / kNCB, c = item % kNCB * CW + lane % CW;
+        const size_t ri = (size_t)grp * R + r;
+        float m = -INFINITY, l = 0.f;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int k0 = sl; k0 < ns; k0 += kSL * kUnroll) {
+            f32x4 ov[kUnroll];
+            float mv[kUnroll], lv[kUnroll];
+    #pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                const int k = min(k0 + u * kSL, ns - 1);
+                const size_t pi = partial(k, r);
+                ov[u] = *reinterpret_cast<const f32x4*>(p.Opart + pi * D + 4 * c);
+                mv[u] = p.Mpart[pi];
+                lv[u] = p.Lpart[pi];
+            }
+            float mx = m;
+    #pragma unroll
+            for (int u = 0; u < kUnroll; ++u) mx = fmaxf(mx, mv[u]);
+            const bool none = mx == -INFINITY;            // weight 0 below keeps a NaN
+            const float keep = none ? 1.f : exp2_hw((m - mx) * kLog2e);
+            acc *= keep;
+            l *= keep;
+    #pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                const bool in = k0 + u * kSL < ns;
+                const float w = in && !none ? exp2_hw((mv[u] - mx) * kLog2e) : 0.f;
+                l += in ? w * lv[u] : 0.f;
+                acc += in ? w * ov[u] : f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+            m = mx;
+        }
+        const float mm = reduce_mod<CW, true>(m);
+        const float w = mm == -INFINITY ? 0.f : exp2_hw((m - mm) * kLog2e);
+        l = reduce_mod<CW, false>(l * w);
+        acc *= w;
+        acc.x = reduce_mod<CW, false>(acc.x);
+        acc.y = reduce_mod<CW, false>(acc.y);
+        acc.z = reduce_mod<CW, false>(acc.z);
+        acc.w = reduce_mod<CW, false>(acc.w);
+        if (sl == 0) {
+            store_out4(p, ri * D + 4 * c, acc * (l > 0.f ? 1.0f / l : 0.f));
+            if (c == 0) store_stats(p, ri, mm, l);
+        }
     }
 }
 
