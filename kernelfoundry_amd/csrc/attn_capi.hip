@@ -116,7 +116,22 @@ constexpr int kWideCausalMinKeys = 2048;
 // 4 x 4096 (2) 18.9 -> 15.8.  16 rows (q_len 4) 16 x 4096 32.8 -> 26.6; with 32
 // rows (MQA) a partial is as large as a stage, and 64 x 4096 keys at D = 64
 // ran 13.6 -> 17.6: not taken.
-constexpr int kRaggedMinShare(int D) { return D == 128 ? 3 : 2; }
+// More where the rows' partials, or a merge launch that the unsplit plan does
+// without, weigh more against a worker's stages: 8 / 1 heads, D = 128 (8 rows)
+// 256 x 1024 keys (4) 19.2 -> 23.6, 64 x 4096 (4) 20.0 -> 21.2; D = 64, 298 x 336
+// at 16 / 2 (2.1) 16.3 -> 19.2; D = 16, 4 / 2 heads 361 x 368 (2.8) 10.1 -> 14.2,
+// 1024 x 256 (5.3) 17.1 -> 17.9, 512 x 1024 (11) 18.6 -> 17.4.  Not where there is
+// a head per worker, of which the split grid makes many rounds (2048 x 128 at
+// 8 / 1, D = 128 (4) 54.5 -> 38.6, 4096 x 64 at 4 / 2, D = 16 (5.3) 54 -> 24), or
+// where splits take it two rounds (58 x 2 x 5152 at 8 / 1, D = 128 (4.6) 29.4 ->
+// 22.1; D = 16, 194 x 512 at 8 / 4 (4) 17.0 -> 13.3).  (Of 8 rows at D = 64 in one
+// round of splits the worst was 9 x 31616 at 8 / 1 (2.9), 13.5 -> 15.3.)
+constexpr int kRaggedMinShare(int D, int rows, bool split, long long heads, long long workers, long long grid,
+                              int cus) {
+    const int least = D == 128 ? 3 : 2;
+    if (heads >= workers || (split && grid >= 2LL * cus)) return least;
+    return D == 16 ? 6 : D == 128 && rows >= 8 ? 5 : D == 64 && !split ? 3 : least;
+}
 constexpr int kRaggedMaxRows = 16;
 // Without key counts the split grid stays where it is one round of workgroups
 // (8 x 4096 keys 26.2 us against 28.6, 1 x 65536 47.2 against 52.7); a head
@@ -400,8 +415,10 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
         // worker and up to kRaggedMaxRows rows per KV head on.
         const long long cap_stages = n_groups * ((kv_len + 31LL) / 32);
         const int wgs = kf::ragged_workgroups(D, cus);
+        const long long workers = (long long)wgs * kf::ragged_waves(D);
+        const int share = kRaggedMinShare(D, (int)R, splits > 1, n_groups, workers, p.grid, cus);
         if (nst == 0 && R <= kRaggedMaxRows && cap_stages <= (1LL << 30) && rows_total * (D / 4) <= INT_MAX &&
-            cap_stages >= (long long)kRaggedMinShare(D) * wgs * kf::ragged_waves(D)) {
+            cap_stages >= share * workers) {
             p.ragged_wgs = wgs;
             p.ragged_parts = (size_t)2 * wgs * kf::ragged_waves(D) * (size_t)R;
             p.ragged_bytes = split_ws_bytes(p.ragged_parts, D) + align_up((size_t)n_groups * sizeof(kf::u32x4), kWsAlign);

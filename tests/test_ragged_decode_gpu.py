@@ -81,8 +81,13 @@ def test_other_calls_keep_their_kernels_and_workspace():
     assert kf.workspace_bytes(12, 1, 4096, 32, 8, 128) == kf.workspace_bytes_lens(12, 1, 4096, 32, 8, 128)
     for B in (8, 16, 32):
         assert "ragged" not in kf.kernel_names(B, 1, 4096, 32, 8, 128)
-    # Small capacities and more than 16 rows per KV head never.
-    for shape in ((4, 1, 4096, 32, 8, 128), (1, 1, 4096, 32, 8, 128), (64, 1, 4096, 32, 1, 64)):
+    # Small capacities and more than 16 rows per KV head never; larger ones for
+    # eight rows and more, and at D = 16, unless there is a head per worker.
+    for shape in ((2048, 1, 128, 8, 1, 128), (4096, 1, 64, 4, 2, 16)):
+        assert "ragged" in kf.kernel_names(*shape, masked=True)
+    for shape in ((4, 1, 4096, 32, 8, 128), (1, 1, 4096, 32, 8, 128), (64, 1, 4096, 32, 1, 64),
+                  (256, 1, 1024, 8, 1, 128), (64, 1, 4096, 8, 1, 128), (298, 1, 336, 16, 2, 64),
+                  (361, 1, 368, 4, 2, 16)):
         assert "ragged" not in kf.kernel_names(*shape, masked=True)
         assert kf.workspace_bytes_lens(*shape) == kf.workspace_bytes(*shape)
     # A workspace of the capacity's plan is enough (the call then ends at
