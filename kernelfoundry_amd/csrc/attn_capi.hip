@@ -139,8 +139,11 @@ constexpr int kRaggedMaxRows = 16;
 // ragged decode: 12 x 4096 keys 44.1 -> 39.8, 20 x 4096 70.1 -> 60.3,
 // 40 x 1000 43.1 -> 35.4, 6 x 4096 29.8 -> 23.7; D = 256 (always two rounds)
 // 8 x 4096 at 16 / 4 heads 37.7 -> 31.7.  Of several rounds the least gain was
-// 24 x 8192 keys, 129.7 -> 130.3.
+// 24 x 8192 keys, 129.7 -> 130.3.  D = 16, whose workgroups share a CU: 19 x
+// 12123 at 4 / 2 heads (3 rounds) 12.3 -> 15.1, 43 x 4252 (3.7) 12.9 -> 13.9, 153
+// x 3624 (6) 21.5 -> 21.5, 132 x 2 x 4078 at 8 / 4 (21) 41.8 -> 33.8.
 constexpr int kRaggedEvenRows = 8;
+constexpr int kRaggedEvenRounds(int D) { return D == 16 ? 5 : 1; }
 // Waves of its merge, beyond which heads of many partials share (25 x 2 queries,
 // 64 / 8 heads: 22.1 us, with 4096 23.8, with 2048 26.8; large batches alike).
 constexpr int kRaggedMergeMaxWaves = 8192;
@@ -423,8 +426,9 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
             p.ragged_parts = (size_t)2 * wgs * kf::ragged_waves(D) * (size_t)R;
             p.ragged_bytes = split_ws_bytes(p.ragged_parts, D) + align_up((size_t)n_groups * sizeof(kf::u32x4), kWsAlign);
             // Equal lengths: where the streaming kernel's grid takes more
-            // than one round of workgroups.
-            p.ragged_even = R <= kRaggedEvenRows && p.n_splits > 1 && p.grid > cus;
+            // than one round of workgroups (kRaggedEvenRounds).
+            p.ragged_even = R <= kRaggedEvenRows && p.n_splits > 1 &&
+                            p.grid > (long long)kRaggedEvenRounds(D) * cus;
         }
     } else {
         // Waves per workgroup: the most the head dimension allows.  When that

@@ -15,6 +15,7 @@ import pytest
 
 import kernelfoundry_amd as kf
 from oracle import attn_oracle as orc
+from tests._parity import run_and_check
 
 
 def _lens(kind, B, cap, seed):
@@ -178,6 +179,74 @@ def test_ragged_parity(case):
         assert np.abs(lse[full] - (Mr[full] + np.log(Lr[full]))).max() <= 1e-3
     # The same rows, rounded once.
     assert np.array_equal(O16.cpu().numpy(), O.astype(np.float16))
+
+
+# Without key counts: equal lengths that end inside a stage, both ways of
+# merging, every head dimension.
+EVEN = [
+    # B, H_q, H_kv, q_len, kv_len, D, causal
+    (132, 8, 4, 2, 4078, 16, True),
+    (108, 8, 4, 1, 1258, 16, False),
+    (25, 16, 16, 1, 777, 64, False),
+    (60, 16, 16, 2, 1487, 64, True),
+    (12, 32, 8, 1, 4099, 128, False),
+    (21, 16, 4, 2, 1001, 256, True),
+]
+
+
+def _even_id(c):
+    return "B{}_Hq{}_Hkv{}_q{}_kv{}_D{}".format(*c[:6])
+
+
+@pytest.mark.parametrize("case", EVEN, ids=_even_id)
+def test_equal_lengths_take_the_ragged_kernel(case):
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("a GPU is visible: the plan is for its CU count")
+    B, H_q, H_kv, q, kv, D, causal = case
+    names = kf.kernel_names(B, q, kv, H_q, H_kv, D, causal=causal)
+    assert names == f"kf_attn_decode_ragged_kernel<{D}, false> + kf_attn_ragged_merge_kernel<{D}>"
+    # At D = 16 only grids of many rounds.
+    assert "ragged" not in kf.kernel_names(19, 1, 12123, 4, 2, 16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", EVEN, ids=_even_id)
+def test_equal_lengths_parity(case):
+    B, H_q, H_kv, q, kv, D, causal = case
+    run_and_check(B, H_q, H_kv, q, kv, D, causal, None, seed=900 + B)
+
+
+@pytest.mark.gpu
+def test_ragged_decode_replayed_with_other_key_counts():
+    """One captured call, replayed several times with other key counts in the
+    same array and eager work between: every replay has the bits of an eager
+    call with those counts (the division is found on the device)."""
+    import torch
+    B, q, cap, H_q, H_kv, D = 16, 1, 4096, 32, 8, 128
+    print("case replay", flush=True)
+    assert "ragged" in kf.kernel_names(B, q, cap, H_q, H_kv, D, masked=True)
+    normal = lambda *s: torch.randn(s, device="cuda", dtype=torch.float16)
+    Q, K, V = normal(B, H_q, q, D), normal(B, H_kv, cap, D), normal(B, H_kv, cap, D)
+    lens = torch.full((B,), cap, dtype=torch.int32, device="cuda")
+    ws = torch.empty(kf.workspace_bytes_lens(B, q, cap, H_q, H_kv, D), dtype=torch.uint8, device="cuda")
+    out = torch.empty((B, H_q, q, D), dtype=torch.float32, device="cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        kf.attn_fwd(Q, K, V, out, kv_lens=lens, workspace=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        kf.attn_fwd(Q, K, V, out, kv_lens=lens, workspace=ws)
+    for kind in ("mixed", "full", "empty", "one_long", "short", "mixed"):
+        lens.copy_(torch.from_numpy(_lens(kind, B, cap, 3)))
+        ref = kf.attn_fwd(Q, K, V, kv_lens=lens)
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref), kind
 
 
 @pytest.mark.gpu
