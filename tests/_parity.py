@@ -7,7 +7,18 @@ import numpy as np
 from oracle import attn_oracle as orc
 
 
-def run_and_check(B, H_q, H_kv, q_len, kv_len, D, causal, kv_lens, seed):
+def capacity_workspace(B, q_len, kv_len, H_q, H_kv, D):
+    """A workspace with which a decode runs by its plan's splits (the short-split
+    or the streaming kernel), also where a larger one has it shared evenly."""
+    import torch
+
+    import kernelfoundry_amd as kf
+
+    n = kf.workspace_bytes_least(B, q_len, kv_len, H_q, H_kv, D)
+    return torch.empty(n, dtype=torch.uint8, device="cuda")
+
+
+def run_and_check(B, H_q, H_kv, q_len, kv_len, D, causal, kv_lens, seed, by_capacity=False):
     import torch
 
     import kernelfoundry_amd as kf
@@ -19,7 +30,8 @@ def run_and_check(B, H_q, H_kv, q_len, kv_len, D, causal, kv_lens, seed):
     q16, k16, v16 = orc.normal_fp16_inputs(B, H_q, H_kv, q_len, kv_len, D, seed)
     Q, K, V = (torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (q16, k16, v16))
     lens = None if kv_lens is None else torch.tensor(kv_lens, dtype=torch.int32, device="cuda")
-    O, Mi, Li = kf.attn_fwd(Q, K, V, return_stats=True, causal=causal, kv_lens=lens)
+    ws = capacity_workspace(B, q_len, kv_len, H_q, H_kv, D) if by_capacity else None
+    O, Mi, Li = kf.attn_fwd(Q, K, V, return_stats=True, causal=causal, kv_lens=lens, workspace=ws)
     torch.cuda.synchronize()
     O, Mi, Li = O.cpu().numpy(), Mi.cpu().numpy(), Li.cpu().numpy()
     Or, Mr, Lr = orc.sdpa(q16, k16, v16, causal=causal, kv_lens=kv_lens)

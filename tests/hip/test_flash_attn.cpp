@@ -18,6 +18,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <random>
 #include <vector>
 
@@ -148,15 +149,21 @@ static bool run_case(int B, int q_len, int kv_len, int H_q, int H_kv, int D, uin
 // The extensions through kf/flash_attn.hpp, checked for exact agreement with
 // the paths above: kf::attn_fwd_ex without masking and with every key count
 // equal to kv_len, paged decode over pages holding the cache rows in order,
-// and an fp16 O equal to the round-to-nearest-even of the fp32 O.  Paged
-// decode always runs the streaming decode kernel; the batch is large enough
-// for the contiguous plan to run it too (same splits, same arithmetic), which
-// the plan check below confirms.
+// and an fp16 O equal to the round-to-nearest-even of the fp32 O.  Twice: by
+// the launchers, whose workspace has all of them run the ragged decode, and by
+// the C ABI with the plan's partials only, which has them run the streaming
+// decode kernel (same splits, same arithmetic each time).
 static bool run_extension_checks() {
     const int B = 12, H_q = 32, H_kv = 8, D = 128, q_len = 1, kv_len = 4096, page = 16;
     kf_attn_plan_t plan;
     if (kf_attn_plan(B, q_len, kv_len, H_q, H_kv, D, &plan) != KF_OK || plan.splits_per_block != 1) {
         std::printf("  FAIL: the contiguous plan no longer uses the streaming decode kernel\n");
+        return false;
+    }
+    char name[256] = "";
+    if (kf_attn_kernel_names(B, q_len, kv_len, H_q, H_kv, D, 0, nullptr, name, sizeof(name)) != KF_OK ||
+        !std::strstr(name, "kf_attn_decode_ragged_kernel")) {
+        std::printf("  FAIL: the launchers no longer use the ragged decode (%s)\n", name);
         return false;
     }
     const int pages = kv_len / page;
@@ -202,33 +209,63 @@ static bool run_extension_checks() {
     HIP_CHECK(hipMemcpy(dtab, table.data(), table.size() * 4, hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(dlen, lens.data(), lens.size() * 4, hipMemcpyHostToDevice));
 
-    HIP_CHECK(launch_flash_attn(dq, dk, dv, dO0, B, q_len, kv_len, H_q, H_kv, D, nullptr));
-    HIP_CHECK(kf::attn_fwd_ex(dq, dk, dv, dO1, B, q_len, kv_len, H_q, H_kv, D, dlen, 0, nullptr));
-    HIP_CHECK(kf::attn_decode_paged(dq, dkp, dvp, dtab, dlen, dO2, B, q_len, H_q, H_kv, D, page,
-                                    pages, B * pages, 0, nullptr));
-    HIP_CHECK(kf::attn_fwd_ex(dq, dk, dv, dO16, B, q_len, kv_len, H_q, H_kv, D, nullptr,
-                              KF_ATTN_OUT_F16, nullptr));
-    HIP_CHECK(hipDeviceSynchronize());
-    std::vector<float> o0(qn), o1(qn), o2(qn);
-    std::vector<uint16_t> o16(qn);
-    HIP_CHECK(hipMemcpy(o0.data(), dO0, qn * 4, hipMemcpyDeviceToHost));
-    HIP_CHECK(hipMemcpy(o1.data(), dO1, qn * 4, hipMemcpyDeviceToHost));
-    HIP_CHECK(hipMemcpy(o2.data(), dO2, qn * 4, hipMemcpyDeviceToHost));
-    HIP_CHECK(hipMemcpy(o16.data(), dO16, qn * 2, hipMemcpyDeviceToHost));
-    for (void* ptr : {(void*)dq, (void*)dk, (void*)dv, (void*)dkp, (void*)dvp, (void*)dtab,
-                      (void*)dlen, (void*)dO0, (void*)dO1, (void*)dO2, (void*)dO16})
-        (void)hipFree(ptr);
-
-    size_t bad_lens = 0, bad_paged = 0, bad_f16 = 0;
-    for (size_t i = 0; i < qn; ++i) {
-        bad_lens += o1[i] != o0[i];
-        bad_paged += o2[i] != o0[i];
-        bad_f16 += o16[i] != kf_oracle_float_to_half(o0[i]);
+    const size_t least = kf_attn_workspace_bytes_least(B, q_len, kv_len, H_q, H_kv, D);
+    void* dws;
+    HIP_CHECK(hipMalloc(&dws, least));
+    std::vector<float> first;
+    bool ok = true;
+    for (int pass = 0; pass < 2; ++pass) {
+        if (pass == 0) {
+            HIP_CHECK(launch_flash_attn(dq, dk, dv, dO0, B, q_len, kv_len, H_q, H_kv, D, nullptr));
+            HIP_CHECK(kf::attn_fwd_ex(dq, dk, dv, dO1, B, q_len, kv_len, H_q, H_kv, D, dlen, 0, nullptr));
+            HIP_CHECK(kf::attn_decode_paged(dq, dkp, dvp, dtab, dlen, dO2, B, q_len, H_q, H_kv, D, page,
+                                            pages, B * pages, 0, nullptr));
+            HIP_CHECK(kf::attn_fwd_ex(dq, dk, dv, dO16, B, q_len, kv_len, H_q, H_kv, D, nullptr,
+                                      KF_ATTN_OUT_F16, nullptr));
+        } else {
+            const auto fwd = [&](void* O, const int* counts, int flags) {
+                return kf::status_to_hip(kf_attn_fwd_ex(dq, dk, dv, O, nullptr, nullptr, B, q_len, kv_len, H_q,
+                                                        H_kv, D, counts, flags, dws, least, nullptr));
+            };
+            HIP_CHECK(fwd(dO0, nullptr, 0));
+            HIP_CHECK(fwd(dO1, dlen, 0));
+            HIP_CHECK(kf::status_to_hip(kf_attn_decode_paged(dq, dkp, dvp, dtab, dlen, dO2, nullptr, nullptr, B,
+                                                             q_len, H_q, H_kv, D, page, pages, B * pages, 0, dws,
+                                                             least, nullptr)));
+            HIP_CHECK(fwd(dO16, nullptr, KF_ATTN_OUT_F16));
+        }
+        HIP_CHECK(hipDeviceSynchronize());
+        std::vector<float> o0(qn), o1(qn), o2(qn);
+        std::vector<uint16_t> o16(qn);
+        HIP_CHECK(hipMemcpy(o0.data(), dO0, qn * 4, hipMemcpyDeviceToHost));
+        HIP_CHECK(hipMemcpy(o1.data(), dO1, qn * 4, hipMemcpyDeviceToHost));
+        HIP_CHECK(hipMemcpy(o2.data(), dO2, qn * 4, hipMemcpyDeviceToHost));
+        HIP_CHECK(hipMemcpy(o16.data(), dO16, qn * 2, hipMemcpyDeviceToHost));
+        size_t bad_lens = 0, bad_paged = 0, bad_f16 = 0;
+        for (size_t i = 0; i < qn; ++i) {
+            bad_lens += o1[i] != o0[i];
+            bad_paged += o2[i] != o0[i];
+            bad_f16 += o16[i] != kf_oracle_float_to_half(o0[i]);
+        }
+        const bool good = bad_lens == 0 && bad_paged == 0 && bad_f16 == 0;
+        std::printf("  B=%d q_len=1 kv_len=%d GQA %d:%d D=%d page=%d %s decode ... %s (differing elements: "
+                    "key counts %zu, paged %zu, fp16 O %zu)\n",
+                    B, kv_len, H_q, H_kv, D, page, pass ? "streaming" : "ragged", good ? "PASS" : "FAIL", bad_lens,
+                    bad_paged, bad_f16);
+        ok = ok && good;
+        if (pass == 0) {
+            first = o0;
+            continue;
+        }
+        // Two kernels, the same result but for the last bits.
+        float most = 0.f;
+        for (size_t i = 0; i < qn; ++i) most = std::max(most, std::fabs(o0[i] - first[i]));
+        if (most > 2e-4f) std::printf("  FAIL: ragged and streaming decode differ by %g\n", most);
+        ok = ok && most <= 2e-4f;
     }
-    const bool ok = bad_lens == 0 && bad_paged == 0 && bad_f16 == 0;
-    std::printf("  B=%d q_len=1 kv_len=%d GQA %d:%d D=%d page=%d ... %s (differing elements: "
-                "key counts %zu, paged %zu, fp16 O %zu)\n",
-                B, kv_len, H_q, H_kv, D, page, ok ? "PASS" : "FAIL", bad_lens, bad_paged, bad_f16);
+    for (void* ptr : {(void*)dq, (void*)dk, (void*)dv, (void*)dkp, (void*)dvp, (void*)dtab, (void*)dlen,
+                      (void*)dO0, (void*)dO1, (void*)dO2, (void*)dO16, dws})
+        (void)hipFree(ptr);
     return ok;
 }
 

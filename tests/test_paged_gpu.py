@@ -19,6 +19,7 @@ import numpy as np
 import pytest
 
 from oracle import attn_oracle as orc
+from tests._parity import capacity_workspace
 
 pytestmark = pytest.mark.gpu
 
@@ -58,12 +59,16 @@ def _oracle(q16, k16, v16, table, lens, page_size, causal):
     return orc.sdpa(q16, K, V, causal=causal, kv_lens=lens, key_valid=valid)
 
 
-def _run(q16, k16, v16, table, lens, causal):
+def _run(q16, k16, v16, table, lens, causal, by_capacity=False):
     import kernelfoundry_amd as kf
     torch = _torch()
+    ws = None
+    if by_capacity:
+        B, H_q, q_len, D = q16.shape
+        ws = capacity_workspace(B, q_len, k16.shape[2] * table.shape[1], H_q, k16.shape[1], D)
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
     O, Mi, Li = kf.attn_decode_paged(t(q16), t(k16), t(v16), t(table), t(lens),
-                                     return_stats=True, causal=causal)
+                                     return_stats=True, causal=causal, workspace=ws)
     torch.cuda.synchronize()
     return O.cpu().numpy(), Mi.cpu().numpy(), Li.cpu().numpy()
 
@@ -94,8 +99,10 @@ PAGED_CASES = [
     (2, 8, 2, 4, 256, 32, 12, [350, 200], True, ()),          # D=256, causal q_len=4
     (2, 32, 8, 1, 128, 16, 64, [1024, 1000], False, [(0, 3, -5), (1, 10, 10 ** 6)]),
     (4, 32, 4, 1, 128, 128, 33, [4200, 3000, 129, 4224], False, ()),
-    # Jobs large enough for the streaming decode kernel (the ones above run
-    # the short-split kernel's paged form), with invalid page ids.
+    # Jobs large enough for the ragged decode, and given a workspace of the
+    # plan's partials for the streaming decode kernel, with invalid page ids
+    # (the ones above run the short-split kernel's paged form, the last of them
+    # the streaming kernel's).
     (12, 32, 8, 1, 128, 16, 256, [4096 - 53 * b for b in range(12)], False,
      [(0, 3, -5), (5, 200, 10 ** 6)]),
     (24, 16, 16, 1, 64, 64, 40, [2560 - 100 * b for b in range(24)], False, [(7, 0, -1)]),
@@ -104,15 +111,21 @@ PAGED_CASES = [
 
 
 def test_paged_cases_reach_both_decode_kernels():
-    """The cases above run the short-split decode kernel's paged form and the
-    streaming kernel's (the planner sizes a paged decode like a contiguous one
-    over the capacity): both appear, both with invalid page ids."""
+    """The cases above run the paged forms of the short-split kernel and, as
+    they are and by the capacity's splits, of the ragged and the streaming
+    decode at D = 64, 128 and 256, with invalid page ids (the planner sizes a
+    paged decode like a contiguous one over the capacity)."""
     import kernelfoundry_amd as kf
     kinds = set()
     for B, H_q, H_kv, q_len, D, ps, max_pages, kv_lens, causal, bad in PAGED_CASES:
-        p = kf.plan(B, q_len, ps * max_pages, H_q, H_kv, D)
-        kinds.add((p.splits_per_block == kf.plan(1, 1, 4096, 32, 8, 128).splits_per_block, bool(bad)))
-    assert kinds >= {(True, True), (False, True), (True, False)}
+        shape = B, q_len, ps * max_pages, H_q, H_kv, D
+        name = kf.kernel_names(*shape, causal=causal, masked=True).split("<")[0]
+        stream = kf.plan(*shape).splits_per_block == 1    # the plan's own kernel
+        assert stream == (name != "kf_attn_decode_short_kernel")
+        kinds.add((name, D if "ragged" in name else 0, bool(bad)))
+    assert kinds >= {("kf_attn_decode_short_kernel", 0, True), ("kf_attn_decode_short_kernel", 0, False),
+                     ("kf_attn_decode_kernel", 0, False)}
+    assert kinds >= {("kf_attn_decode_ragged_kernel", D, True) for D in (64, 128, 256)}
 
 
 @pytest.mark.parametrize("case", PAGED_CASES, ids=lambda c: "B{}_Hq{}_Hkv{}_q{}_D{}_ps{}_{}{}".format(
@@ -125,8 +138,9 @@ def test_paged_decode_parity(case):
     q16, k16, v16, table, lens = _paged_inputs(B, H_q, H_kv, q_len, D, ps, max_pages, num_pages,
                                                kv_lens, 900 + D + ps, bad)
     ref = _oracle(q16, k16, v16, table, lens, ps, causal)
-    got = _run(q16, k16, v16, table, lens, causal)
-    _check(got, ref, f"case {case}")
+    for by_capacity in (False, True):
+        got = _run(q16, k16, v16, table, lens, causal, by_capacity)
+        _check(got, ref, f"case {case} by_capacity={by_capacity}")
 
 
 @pytest.mark.parametrize("page_size", [16, 32, 64])
@@ -163,13 +177,14 @@ def test_paged_short_split_in_order_equals_contiguous_bitwise(page_size):
 def test_paged_in_order_equals_contiguous_bitwise(page_size):
     """Pages holding the rows of a contiguous cache in order: the paged kernel
     computes exactly what kf_attn_fwd_ex computes on the contiguous cache
-    (same splits, same stages, same arithmetic).  The batch is large enough
-    for the streaming decode kernel on both."""
+    (same splits, same stages, same arithmetic): the ragged decode on both,
+    and given a workspace of the plan's partials the streaming decode."""
     import kernelfoundry_amd as kf
     torch = _torch()
     B, H_q, H_kv, D, max_pages = 12, 32, 8, 128, 4096 // page_size
     cap = max_pages * page_size
     assert kf.plan(B, 1, cap, H_q, H_kv, D).splits_per_block == 1
+    assert "decode_ragged" in kf.kernel_names(B, 1, cap, H_q, H_kv, D, masked=True)
     _announce(test="paged_vs_contiguous", page_size=page_size)
     q16, k16, v16 = orc.normal_fp16_inputs(B, H_q, H_kv, 1, cap, D, 314)
     to_pages = lambda a: a.reshape(B, H_kv, max_pages, page_size, D).transpose(0, 2, 1, 3, 4) \
@@ -177,7 +192,11 @@ def test_paged_in_order_equals_contiguous_bitwise(page_size):
     table = np.arange(B * max_pages, dtype=np.int32).reshape(B, max_pages)
     lens = np.array([cap - 37 * b for b in range(B)], dtype=np.int32)
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
-    Op = kf.attn_decode_paged(t(q16), t(to_pages(k16)), t(to_pages(v16)), t(table), t(lens))
-    Oc = kf.attn_fwd(t(q16), t(k16), t(v16), kv_lens=t(lens))
-    torch.cuda.synchronize()
-    assert torch.equal(Op, Oc)
+    outs = []
+    for ws in (None, capacity_workspace(B, 1, cap, H_q, H_kv, D)):
+        Op = kf.attn_decode_paged(t(q16), t(to_pages(k16)), t(to_pages(v16)), t(table), t(lens), workspace=ws)
+        Oc = kf.attn_fwd(t(q16), t(k16), t(v16), kv_lens=t(lens), workspace=ws)
+        torch.cuda.synchronize()
+        assert torch.equal(Op, Oc)
+        outs.append(Oc)
+    assert not torch.equal(*outs)   # two kernels

@@ -17,6 +17,7 @@ import numpy as np
 import pytest
 
 from oracle import attn_oracle as orc
+from tests._parity import capacity_workspace
 
 pytestmark = pytest.mark.gpu
 
@@ -128,7 +129,9 @@ def test_parity_with_stats(case):
                                                          (12, 2, 1500, True, True)])
 def test_d256_streaming_decode(B, q_len, kv_len, causal, ragged):
     """D = 256 on the streaming decode kernel (Q^T fragments read from LDS at
-    every stage), with its split merge; key counts and causal masking."""
+    every stage), with its split merge: a workspace of the plan's partials;
+    key counts and causal masking.  And as the call runs by itself, on the
+    ragged decode."""
     import kernelfoundry_amd as kf
     torch = _torch()
     H_q, H_kv, D = 16, 4, 256
@@ -139,11 +142,15 @@ def test_d256_streaming_decode(B, q_len, kv_len, causal, ragged):
     lens = [kv_len - 97 * b for b in range(B)] if ragged else None
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
     kv_t = torch.tensor(lens, dtype=torch.int32, device="cuda") if ragged else None
-    O, Mi, Li = kf.attn_fwd(t(q16), t(k16), t(v16), return_stats=True, causal=causal, kv_lens=kv_t)
-    torch.cuda.synchronize()
+    assert "decode_ragged" in kf.kernel_names(B, q_len, kv_len, H_q, H_kv, D, causal=causal, masked=ragged)
+    ws = capacity_workspace(B, q_len, kv_len, H_q, H_kv, D)
     Or, Mr, Lr = orc.sdpa(q16, k16, v16, causal=causal, kv_lens=lens)
-    _check(O.cpu().numpy(), Or, "D=256 streaming decode")
-    _check_stats(Mi.cpu().numpy(), Li.cpu().numpy(), Mr, Lr, "D=256 streaming decode")
+    for what, workspace in (("streaming", ws), ("ragged", None)):
+        O, Mi, Li = kf.attn_fwd(t(q16), t(k16), t(v16), return_stats=True, causal=causal, kv_lens=kv_t,
+                                workspace=workspace)
+        torch.cuda.synchronize()
+        _check(O.cpu().numpy(), Or, f"D=256 {what} decode")
+        _check_stats(Mi.cpu().numpy(), Li.cpu().numpy(), Mr, Lr, f"D=256 {what} decode")
 
 
 @pytest.mark.parametrize("q_len", [1, 5, 40])

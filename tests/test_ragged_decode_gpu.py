@@ -7,7 +7,7 @@ inside one worker's share, more than 64 and 192 sequences (the batch map's
 registers), more than 256 and 4096 (its blocks, of 64 and 128), counts past the capacity, 1 to 16 rows per KV head (both ways of
 merging), every head dimension, page sizes from 16 rows, invalid page ids.
 Bar as in the other parity tests (fp64 oracle), and the same call by the
-capacity's splits (a workspace of only kf_attn_workspace_bytes) within 2e-4:
+capacity's splits (a workspace of only those partials) within 2e-4:
 P is rounded to fp16 against other row maxima, 2^-11 of values of order 1.
 """
 import numpy as np
@@ -15,7 +15,7 @@ import pytest
 
 import kernelfoundry_amd as kf
 from oracle import attn_oracle as orc
-from tests._parity import run_and_check
+from tests._parity import capacity_workspace, run_and_check
 
 
 def _lens(kind, B, cap, seed):
@@ -144,7 +144,8 @@ def test_ragged_parity(case):
                                         causal=causal)
         kc, valid = orc.paged_to_contiguous(kp, table, ps)
         vc, _ = orc.paged_to_contiguous(vp, table, ps)
-        by_capacity = None
+        by_capacity = kf.attn_decode_paged(Q, K, V, T, L, causal=causal,
+                                           workspace=capacity_workspace(B, q, cap, H_q, H_kv, D))
     else:
         kc, vc = (rng.standard_normal((B, H_kv, cap, D), dtype=np.float32).astype(np.float16)
                   for _ in range(2))
@@ -163,8 +164,7 @@ def test_ragged_parity(case):
     torch.cuda.synchronize()
     Or, Mr, Lr = orc.sdpa(q16, kc, vc, causal=causal, kv_lens=[int(x) for x in used],
                           **({"key_valid": valid} if valid is not None else {}))
-    if by_capacity is not None:
-        assert (O - by_capacity).abs().max().item() <= 2e-4 * max(1.0, np.abs(Or).max())
+    assert (O - by_capacity).abs().max().item() <= 2e-4 * max(1.0, np.abs(Or).max())
     O, Mi, Li, lse = (x.cpu().numpy() for x in (O, Mi, Li, lse))
     assert np.isfinite(O).all()
     empty = np.isneginf(Mr)

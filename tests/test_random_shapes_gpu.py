@@ -3,7 +3,7 @@
 Shapes, masks and output formats are drawn from a fixed seed so that, taken
 together, they cross every dispatch the planner makes: the short-split decode
 kernel (32- and 64-key splits) and the streaming decode kernel, each with and
-without the split merge, and the prefill kernel in every workgroup layout
+without the split merge, the ragged decode, and the prefill kernel in every workgroup layout
 (8 waves x 256 rows, two KV groups of 8 or 4 waves, four KV groups of 8
 waves, 4 and 2 waves; D = 256 with 4 waves) and the wide prefill kernel (8
 waves x 64 rows at D = 64 / 128, 8 x 32 at D = 256, and at D = 256 its two
@@ -93,14 +93,15 @@ CASES = _cases()
 
 def _layout(kf, B, H_q, H_kv, q_len, kv_len, D, causal=False, masked=False):
     """(path, kernel) for decode, kernel "short32" / "short64" (one wave per
-    split of that many keys) or "stream"; ("prefill", waves, kv_groups) for
+    split of that many keys), "stream" or "ragged"; ("prefill", waves, kv_groups) for
     prefill, read from the kernel name (kf_attn_prefill_kernel<D, mask,
     waves, kv_groups>), or ("prefill", "wide", kv_groups) for
     kf_attn_prefill_wide_kernel<D, mask, kv_groups, causal two-block layout>."""
     p = kf.plan(B, q_len, kv_len, H_q, H_kv, D)
-    if p.path not in ("prefill", "prefill_split"):
-        return (p.path, f"short{p.kv_per_split}" if p.splits_per_block == 4 else "stream")
     name = kf.kernel_names(B, q_len, kv_len, H_q, H_kv, D, causal=causal, masked=masked)
+    if p.path not in ("prefill", "prefill_split"):
+        return (p.path, f"short{p.kv_per_split}" if "decode_short" in name else
+                "ragged" if "decode_ragged" in name else "stream")
     if p.path == "prefill_split":
         name = name.split(" + ")[0]
         if name.startswith("kf_attn_prefill_parts_kernel"):
@@ -118,7 +119,7 @@ def test_sweep_covers_every_dispatch():
     import kernelfoundry_amd as kf
     seen = {_layout(kf, *c[:7], c[7] is not None) for c in CASES}
     want = {("decode", "short32"), ("decode_split", "short32"), ("decode_split", "short64"),
-            ("decode", "stream"), ("decode_split", "stream"),
+            ("decode", "stream"), ("decode_split", "stream"), ("decode_split", "ragged"),
             ("prefill", 8, 1), ("prefill", 8, 2), ("prefill", 8, 4), ("prefill", 4, 2), ("prefill", 4, 1),
             ("prefill", 2, 1), ("prefill", "wide", 1), ("prefill", "wide", 2),
             ("prefill_split", 8, 4), ("prefill_split", 2, 1), ("prefill_split", "parts")}
@@ -130,4 +131,7 @@ def test_sweep_covers_every_dispatch():
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "B{}_Hq{}_Hkv{}_q{}_kv{}_D{}_c{}_{}".format(
     c[0], c[1], c[2], c[3], c[4], c[5], int(c[6]), "lens" if c[7] is not None else "full"))
 def test_random_shape_parity(case):
+    import kernelfoundry_amd as kf
     run_and_check(*case)
+    if _layout(kf, *case[:7], case[7] is not None)[1] == "ragged":
+        run_and_check(*case, by_capacity=True)       # and by the plan's splits
