@@ -22,9 +22,10 @@ ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 # Packed-fp32 VALU ops are kept out of every code object (-packed-fp32-ops).
-# -fno-honor-nans lets fmaxf skip NaN canonicalisation of MFMA results (the
-# kernels never produce or test NaN); infinities keep their IEEE meaning,
-# which the -inf score masking relies on.
+# -fno-honor-nans lets fmaxf skip NaN canonicalisation of MFMA results: the
+# kernels never produce or test NaN from finite inputs, and promise nothing
+# for a NaN among them.  Infinities keep their IEEE meaning, which the -inf
+# score masking relies on.
 DEVICE_FLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",

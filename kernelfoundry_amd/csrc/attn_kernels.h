@@ -2863,8 +2863,7 @@ void kf_attn_decode_ragged_kernel(AttnParams p) {
 #pragma unroll
             for (int w = 0; w < NW; ++w)
                 if (w >= w0 && w < w1) {
-                    // Weight 0 for a row without a key here, whose sums are 0
-                    // (NaN if all of its scores were, which stays).
+                    // Weight 0 for a row without a key here, whose sums are 0.
                     const float wt = mw[w] == -INFINITY ? 0.f : exp2_hw((mw[w] - m) * kLog2e);
                     l += wt * lw[w];
                     acc += wt * ow[w];
@@ -2944,7 +2943,7 @@ void kf_attn_ragged_merge_kernel(AttnParams p) {
 #pragma unroll
                 for (int k = 0; k < kRaggedFew; ++k) {
                     const bool in = k < ns;
-                    const float w = in && m != -INFINITY ? exp2_hw((mv[k] - m) * kLog2e) : 0.f;  // 0 keeps a NaN
+                    const float w = in && m != -INFINITY ? exp2_hw((mv[k] - m) * kLog2e) : 0.f;
                     l += in ? w * lv[k] : 0.f;
                     acc += in ? w * ov[k] : f32x4{0.f, 0.f, 0.f, 0.f};
                 }
@@ -2975,7 +2974,7 @@ void kf_attn_ragged_merge_kernel(AttnParams p) {
             float mx = m;
     #pragma unroll
             for (int u = 0; u < kUnroll; ++u) mx = fmaxf(mx, mv[u]);
-            const bool none = mx == -INFINITY;            // weight 0 below keeps a NaN
+            const bool none = mx == -INFINITY;
             const float keep = none ? 1.f : exp2_hw((m - mx) * kLog2e);
             acc *= keep;
             l *= keep;

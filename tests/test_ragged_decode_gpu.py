@@ -255,7 +255,8 @@ def test_ragged_infinity_and_nan(B, q, ps):
     """An infinity in a sequence's last V row, in a stage that other rows do
     not fill, stays one and does not become NaN (0 times it; paged calls:
     contiguous ones repeat that row), a query row of NaN gives NaN and no
-    other row does.  q = 1 and 4: partials straight to memory and by LDS."""
+    other row does.  (The build does not honour NaNs, so that is what this
+    compiler makes of the merges and no promise.)  q = 1 and 4: partials straight to memory and by LDS."""
     import torch
     H_q, H_kv, cap, D = 32, 8, 4096, 128
     print("case", B, q, ps, flush=True)
