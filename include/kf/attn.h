@@ -79,14 +79,19 @@ typedef struct kf_attn_plan_t {
     int kv_per_split;      /* KV rows per partition                             */
     int grid_blocks;       /* workgroups of the main kernel                     */
     int block_threads;     /* threads per workgroup of the main kernel          */
-    size_t workspace_bytes;/* kf_attn_workspace_bytes()                          */
+    size_t workspace_bytes;/* kf_attn_workspace_bytes(): may be more than this
+                              plan's partials, see kf_attn_plan                 */
     int splits_per_block;  /* decode: KV partitions per workgroup (4 = the
                               short-split kernel, one partition per wave;
                               1 = the streaming decode kernel); 0 on prefill    */
 } kf_attn_plan_t;
 
-/* Describe the dispatch kf_attn_fwd would use on the device current on the
- * calling thread.  Validates like kf_attn_fwd (sizes only, no pointers).
+/* Describe the dispatch of an unmasked kf_attn_fwd call on the device current
+ * on the calling thread.  A decode that kf_attn_kernel_names names the ragged
+ * decode for has no fixed partitions; it is described as it runs with less
+ * workspace than that takes, by num_splits partitions of kv_per_split keys on
+ * the streaming decode kernel.  Causal calls and calls with key counts may
+ * take other layouts: kf_attn_kernel_names tells.  Validates like kf_attn_fwd (sizes only, no pointers).
  * The plan is sized for that device's compute units and XCDs, read once per
  * device with hipDeviceGetAttribute (the reference's launcher likewise sizes
  * its launch from the device, tests/test_flash_attn.cu:28-48); without a
@@ -104,11 +109,12 @@ int kf_attn_plan_for_cus(int B, int q_len, int kv_len, int H_q, int H_kv, int D,
                          kf_attn_plan_t* plan);
 
 /* Names of the kernels kf_attn_fwd_ex launches for this shape on the current
- * device, in launch order and as a profiler lists them, e.g.
+ * device given its best workspace (kf_attn_workspace_bytes, or _lens with
+ * kv_lens), in launch order and as a profiler lists them, e.g.
  * "kf_attn_prefill_kernel<128, false, 8, 1>" or
  * "kf_attn_decode_short_kernel<128, 1> + kf_attn_split_merge_kernel<128, 8, 4>";
  * `flags` (KF_ATTN_CAUSAL) and whether kv_lens is non-NULL (never read) pick
- * the masked prefill.  NUL-terminated into buf; KF_ERR_SIZE if buf_bytes is
+ * the masked prefill and its layout, and kv_lens the ragged decode.  NUL-terminated into buf; KF_ERR_SIZE if buf_bytes is
  * too small.  No reference counterpart (its launchers print the launch
  * geometry, tests/test_flash_attn.cu:86-91). */
 int kf_attn_kernel_names(int B, int q_len, int kv_len, int H_q, int H_kv, int D, int flags,
@@ -126,9 +132,13 @@ size_t kf_attn_workspace_bytes(int B, int q_len, int kv_len, int H_q, int H_kv, 
 /* Bytes of workspace with which a kf_attn_fwd_ex call with kv_lens runs its
  * fastest: at least kf_attn_workspace_bytes().  A large decode then shares the
  * keys that the sequences really hold evenly over the compute units, instead
- * of splitting every sequence by the kv_len rows allocated; a call given only
- * kf_attn_workspace_bytes() still runs, by those splits (the two differ in
- * the last bits, within the same tolerance).  No reference counterpart. */
+ * of splitting every sequence by the kv_len rows allocated; a call given less,
+ * down to kf_attn_workspace_bytes_least(), still runs, by those splits (the
+ * two differ in the last bits, within the same tolerance).  Shared evenly, a
+ * sequence's keys are cut where the shares end, so its last bits depend on the
+ * other sequences' key counts; by the splits they depend on the shape alone.
+ * Sequences that all fill their kv_len rows run up to about a tenth faster by
+ * the splits where those take one round.  No reference counterpart. */
 size_t kf_attn_workspace_bytes_lens(int B, int q_len, int kv_len, int H_q, int H_kv, int D);
 
 /* Bytes of workspace that a caller who has any should give this shape at
@@ -179,9 +189,9 @@ int kf_attn_fwd(const void* Q, const void* K, const void* V, float* O,
  * KF_ATTN_OUT_BF16 (then 2-byte elements, still 16-byte aligned; the
  * reference's PyTorch comparator outputs fp16, bench_flash_attn2.py:11-12);
  * KF_ATTN_LSE replaces the (Mi, Li) pair by one log-sum-exp per row in
- * row_max.  KF_ATTN_OUT_F16 | KF_ATTN_OUT_BF16 -> KF_ERR_FLAGS.  Shapes, workspace
- * and the kernels chosen are those of kf_attn_fwd (kf_attn_plan,
- * kf_attn_workspace_bytes apply unchanged). */
+ * row_max.  KF_ATTN_OUT_F16 | KF_ATTN_OUT_BF16 -> KF_ERR_FLAGS.  Shapes and the
+ * workspace needed are those of kf_attn_fwd (kf_attn_workspace_bytes; with
+ * kv_lens a decode runs faster given kf_attn_workspace_bytes_lens). */
 int kf_attn_fwd_ex(const void* Q, const void* K, const void* V, void* O,
                    float* row_max, float* row_sumexp,
                    int B, int q_len, int kv_len, int H_q, int H_kv, int D,

@@ -981,8 +981,9 @@ int describe_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const 
     plan->rows_per_group = pl.R;
     plan->num_splits = pl.n_splits;
     plan->kv_per_split = pl.kv_per_split;
-    // The unmasked dispatch (kf_attn_fwd); causal calls of kf_attn_fwd_ex
-    // run the 256-row kernel's grid at D = 64 / 128 and this grid at D = 256.
+    // The unmasked dispatch (kf_attn_fwd) by the plan's splits; causal calls
+    // may run the 256-row kernel's grid or a layout of plan_causal, decodes with
+    // their best workspace the ragged kernel's.
     plan->grid_blocks = pl.wide_row_tiles > 0 ? pl.wide_grid : pl.grid;
     plan->block_threads = pl.wide_row_tiles > 0 ? kf::WideCfg<128>::kThreads : pl.threads;
     plan->workspace_bytes = best_ws_bytes(pl, false);
@@ -1198,7 +1199,7 @@ const char* kf_status_string(int status) {
         case KF_ERR_GQA: return "H_q must be a positive multiple of H_kv";
         case KF_ERR_SIZE: return "invalid size (non-positive or beyond 32-bit in-head indexing)";
         case KF_ERR_NULL: return "required pointer is NULL";
-        case KF_ERR_WORKSPACE: return "workspace missing or smaller than kf_attn_workspace_bytes()";
+        case KF_ERR_WORKSPACE: return "workspace missing or smaller than the plan's partials (kf_attn_workspace_bytes_least())";
         case KF_ERR_ALIGN: return "device pointer not 16-byte aligned (workspace: 256-byte)";
         case KF_ERR_HIP: return "HIP runtime error (see kf_last_hip_error)";
         case KF_ERR_FLAGS: return "unknown or conflicting flag bits (KF_ATTN_CAUSAL, KF_ATTN_OUT_F16 or KF_ATTN_OUT_BF16, KF_ATTN_LSE)";

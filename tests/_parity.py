@@ -15,6 +15,8 @@ def capacity_workspace(B, q_len, kv_len, H_q, H_kv, D):
     import kernelfoundry_amd as kf
 
     n = kf.workspace_bytes_least(B, q_len, kv_len, H_q, H_kv, D)
+    if "decode_ragged" in kf.kernel_names(B, q_len, kv_len, H_q, H_kv, D, masked=True):
+        assert n < kf.workspace_bytes_lens(B, q_len, kv_len, H_q, H_kv, D)
     return torch.empty(n, dtype=torch.uint8, device="cuda")
 
 

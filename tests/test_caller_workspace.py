@@ -1,6 +1,7 @@
 """The caller's workspace in the Python entries: used whenever the call runs
 with it, refused only where the call cannot do without one and the buffer is
 no workspace (another device, not contiguous)."""
+import numpy as np
 import pytest
 
 import kernelfoundry_amd as kf
@@ -27,6 +28,34 @@ def test_least_workspace(shape, splits):
     assert kf.workspace_bytes_least(*shape) == up(4 * parts * D) + 2 * up(4 * parts)
     assert kf.workspace_bytes_least(*shape) <= kf.workspace_bytes(*shape) <= kf.workspace_bytes_lens(*shape)
     assert kf.workspace_bytes_least(1, 1, 1, 3, 2, 128) == 0   # invalid
+
+
+def test_plan_describes_the_call_given_its_partials():
+    """kf_attn_plan and kf_attn_kernel_names: a decode that is named by the
+    ragged decode is described by the splits it runs with less workspace, all
+    others by the plan's own kernel and the workspace it asks for."""
+    rng = np.random.default_rng(5)
+    up = lambda n: -(-n // 256) * 256
+    seen = set()
+    for _ in range(400):
+        D = int(rng.choice([16, 64, 128, 256]))
+        H_kv = int(rng.choice([1, 2, 4, 8, 16]))
+        H_q = H_kv * int(rng.choice([1, 2, 4, 8]))
+        shape = B, q, kv, *_ = (int(2 ** rng.uniform(0, 8)), int(rng.integers(1, 5)), int(2 ** rng.uniform(5, 15)),
+                                H_q, H_kv, D)
+        p = kf.plan(*shape)
+        least = kf.workspace_bytes_least(*shape)
+        parts = p.num_splits * B * H_q * q if p.num_splits > 1 else 0
+        assert p.workspace_bytes == kf.workspace_bytes(*shape) >= least
+        if p.path not in ("decode", "decode_split"):
+            continue
+        assert least == up(4 * parts * D) + 2 * up(4 * parts)
+        ragged = "decode_ragged" in kf.kernel_names(*shape)
+        assert ragged or p.workspace_bytes == least
+        assert not ragged or (p.path == "decode_split" and p.splits_per_block == 1)
+        assert ("decode_short" in kf.kernel_names(*shape)) == (p.splits_per_block == 4)
+        seen.add((ragged, p.path))
+    assert {(True, "decode_split"), (False, "decode_split"), (False, "decode")} <= seen
 
 
 def test_the_callers_buffer_is_taken_where_the_call_runs_with_it():
