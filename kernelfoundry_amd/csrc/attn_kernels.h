@@ -218,11 +218,18 @@ __device__ __forceinline__ void store_stats(const AttnParams& p, size_t r, float
     }
 }
 
+// A wave-uniform element of an array that no kernel writes, by a scalar load
+// (the compiler falls back to a vector load, and its in-order wait for every
+// copy in flight, where the kernel's own stores, or an asm statement, might alias).
+__device__ __forceinline__ int uniform_load(const int* a, int i) {
+    return ((const __attribute__((address_space(4))) int*)a)[i];
+}
+
 // Keys of the sequence that KV-head group `grp` belongs to, clamped to
 // [0, kv_len].
 __device__ __forceinline__ int batch_kv_len(const AttnParams& p, int grp) {
     if (!p.kv_lens) return p.kv_len;
-    return min(max(p.kv_lens[grp / p.heads_kv], 0), p.kv_len);
+    return min(max(uniform_load(p.kv_lens, grp / p.heads_kv), 0), p.kv_len);
 }
 
 // Number of leading keys visible to query index qi (0 <= qi < q_len) of a
@@ -2321,13 +2328,6 @@ constexpr int kRaggedSpreadRows = 8;      // query rows per KV head
 constexpr int kRaggedSpreadStages = 12;   // stages per worker
 constexpr int kRaggedSpreadParts = 32;    // partials of an average head: one trip of the merge
 inline int ragged_waves(int D) { return D == 128 ? RaggedCfg<128>::kWaves : RaggedCfg<64>::kWaves; }
-
-// A wave-uniform element of an array that no kernel writes, by a scalar load
-// (the compiler falls back to a vector load, and its in-order wait for every
-// copy in flight, where the kernel's own stores might alias).
-__device__ __forceinline__ int uniform_load(const int* a, int i) {
-    return ((const __attribute__((address_space(4))) int*)a)[i];
-}
 
 // The kernel's parameter block re-read from the kernel arguments: for what a
 // long loop does not need, so that it holds no scalar registers there.
