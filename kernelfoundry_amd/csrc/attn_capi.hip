@@ -124,15 +124,25 @@ constexpr int kWideCausalMinKeys = 2048;
 // a head per worker, of which the split grid makes many rounds (2048 x 128 at
 // 8 / 1, D = 128 (4) 54.5 -> 38.6, 4096 x 64 at 4 / 2, D = 16 (5.3) 54 -> 24), or
 // where splits take it two rounds (58 x 2 x 5152 at 8 / 1, D = 128 (4.6) 29.4 ->
-// 22.1; D = 16, 194 x 512 at 8 / 4 (4) 17.0 -> 13.3).  (Of 8 rows at D = 64 in one
-// round of splits the worst was 9 x 31616 at 8 / 1 (2.9), 13.5 -> 15.3.)
-constexpr int kRaggedMinShare(int D, int rows, bool split, long long heads, long long workers, long long grid,
-                              int cus) {
+// 22.1; D = 16, 194 x 512 at 8 / 4 (4) 17.0 -> 13.3).  D = 64, 8 rows, many splits
+// in one round: 9 x 31616 at 8 / 1 (2.9) 13.5 -> 15.3, 18 x 2 x 9792 at 16 / 2 (3.6)
+// 15.4 -> 16.8.
+constexpr int kRaggedMinShare(int D, int rows, long long splits, long long heads, long long workers,
+                              long long grid, int cus) {
     const int least = D == 128 ? 3 : 2;
-    if (heads >= workers || (split && grid >= 2LL * cus)) return least;
-    return D == 16 ? 6 : D == 128 && rows >= 8 ? 5 : D == 64 && !split ? 3 : least;
+    if (heads >= workers || (splits > 1 && grid >= 2LL * cus)) return least;
+    if (D == 64 && rows >= 8 && splits >= 7 && grid <= cus) return 5;
+    return D == 16 ? 6 : D == 128 && rows >= 8 ? 5 : D == 64 && splits == 1 ? 3 : least;
 }
 constexpr int kRaggedMaxRows = 16;
+// From so many rows on, an unsplit grid of up to three rounds keeps the plan:
+// its one launch merges nothing.  Spread lengths gained little, full ones lost:
+// 28 x 4 x 1984 at 24 / 8 heads, D = 128 (12 rows) 29.7 -> 25.6 us and 38.7 ->
+// 45.7, 31 x 2 x 3360 at 32 / 8, D = 64 (8) 24.6 -> 23.4 and 35.4 -> 44.0, 121 x
+// 1152 at 28 / 4 (7) 32.9 -> 32.0 and 50.7 -> 55.1.  Taken: 4 rows, 32 x 2048 at
+// 32 / 8, 29.5 -> 24.1 and 43.6 -> 48.4; more rounds, 190 x 4 x 720 at 16 / 8 (8
+// rows) 63.4 -> 56.6 and 111.6 -> 109.6.
+constexpr int kRaggedUnsplitRows = 7;
 // Without key counts the split grid stays where it is one round of workgroups
 // (8 x 4096 keys 26.2 us against 28.6, 1 x 65536 47.2 against 52.7); a head
 // count that takes it several (each with its prologue and merge) goes to the
@@ -419,8 +429,9 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
         const long long cap_stages = n_groups * ((kv_len + 31LL) / 32);
         const int wgs = kf::ragged_workgroups(D, cus);
         const long long workers = (long long)wgs * kf::ragged_waves(D);
-        const int share = kRaggedMinShare(D, (int)R, splits > 1, n_groups, workers, p.grid, cus);
-        if (nst == 0 && R <= kRaggedMaxRows && cap_stages <= (1LL << 30) && rows_total * (D / 4) <= INT_MAX &&
+        const int share = kRaggedMinShare(D, (int)R, splits, n_groups, workers, p.grid, cus);
+        const bool one_launch = splits == 1 && R >= kRaggedUnsplitRows && D <= 128 && p.grid <= 3LL * cus;
+        if (nst == 0 && R <= kRaggedMaxRows && !one_launch && cap_stages <= (1LL << 30) && rows_total * (D / 4) <= INT_MAX &&
             cap_stages >= share * workers) {
             p.ragged_wgs = wgs;
             p.ragged_parts = (size_t)2 * wgs * kf::ragged_waves(D) * (size_t)R;

@@ -88,7 +88,7 @@ def test_other_calls_keep_their_kernels_and_workspace():
         assert "ragged" in kf.kernel_names(*shape, masked=True)
     for shape in ((4, 1, 4096, 32, 8, 128), (1, 1, 4096, 32, 8, 128), (64, 1, 4096, 32, 1, 64),
                   (256, 1, 1024, 8, 1, 128), (64, 1, 4096, 8, 1, 128), (298, 1, 336, 16, 2, 64),
-                  (361, 1, 368, 4, 2, 16)):
+                  (361, 1, 368, 4, 2, 16), (9, 1, 31616, 8, 1, 64), (28, 4, 1984, 24, 8, 128)):
         assert "ragged" not in kf.kernel_names(*shape, masked=True)
         assert kf.workspace_bytes_lens(*shape) == kf.workspace_bytes(*shape)
     # A workspace of the capacity's plan is enough (the call then ends at
