@@ -431,8 +431,8 @@ int make_plan(int B, int q_len, int kv_len, int H_q, int H_kv, int D, const Devi
         const long long workers = (long long)wgs * kf::ragged_waves(D);
         const int share = kRaggedMinShare(D, (int)R, splits, n_groups, workers, p.grid, cus);
         const bool one_launch = splits == 1 && R >= kRaggedUnsplitRows && D <= 128 && p.grid <= 3LL * cus;
-        if (nst == 0 && R <= kRaggedMaxRows && !one_launch && cap_stages <= (1LL << 30) && rows_total * (D / 4) <= INT_MAX &&
-            cap_stages >= share * workers) {
+        if (nst == 0 && R <= kRaggedMaxRows && !one_launch && cap_stages >= share * workers &&
+            cap_stages <= (1LL << 30) && rows_total * (D / 4) <= INT_MAX) {
             p.ragged_wgs = wgs;
             p.ragged_parts = (size_t)2 * wgs * kf::ragged_waves(D) * (size_t)R;
             p.ragged_bytes = split_ws_bytes(p.ragged_parts, D) + align_up((size_t)n_groups * sizeof(kf::u32x4), kWsAlign);
@@ -636,10 +636,10 @@ hipError_t launch_prefill_kernel(const Plan& plan, const kf::AttnParams& params,
         }
         // The order of the row tiles.  The divisions of causal_place and
         // causal_tile take up to 0.7 us of a call, so a grid of one round, heads of
-        // a tile or so in up to two and rows that see nearly equal counts go from each KV
-        // head's last tile down, and so does one query head per KV head, for which
-        // that is causal_tile's order (4 x 576 queries at 16 / 16 heads, D = 64
-        // 17.9 us by causal_tile, 17.3 so; 2 x 100 at 32 / 8, D = 128 7.50, 7.33).
+        // a tile or so in up to two rounds, and rows that see nearly equal counts go
+        // from each KV head's last tile down, and so does one query head per KV head,
+        // for which that is causal_tile's order (4 x 576 queries at 16 / 16 heads,
+        // D = 64 17.9 us by causal_tile, 17.3 so; 2 x 100 at 32 / 8, D = 128 7.50, 7.33).
         // 8 x 500 at 32 / 8 heads, D = 128 48.5 so, 44.2 by causal_tile.
         const int grid = std::max(pl.grid, pl.wide_row_tiles > 0 ? pl.wide_grid : 0);
         if (grid > pl.cus) {
